@@ -1756,14 +1756,51 @@ __host__ __device__ constexpr int64_t map_row_words(int vocab) {
     return static_cast<int64_t>((vocab + kMapTile - 1) / kMapTile) * kMapSub * kMapPartWords;
 }
 
+// The exponent whose binade holds the sequential sum that S approximates (the
+// two differ by far less than 2^-20), or the one above.
+__device__ __forceinline__ int sum_exp(double S) { return exp_of(S * (1.0 + 0x1p-20)); }
+
+// Whether the reciprocal 1 / den rounds to the same float for every value that
+// the reference's sequential double sum can have, S being a sum of the same
+// terms in another order: then no replay is needed, as only that float is
+// used (generation.cpp:98-101). With e = sum_exp(S) and U = 2^(e-52), a term
+// whose lowest set bit is at least U adds without rounding except where the
+// sum enters a higher binade (the sum starts at exp(0) = 1, so at most e
+// times); a float at or above 2^(e-29) is such a term. Each other term
+// (`fine` of them, or more) rounds by at most U / 2. The parallel sum adds at
+// most V / 512 + 512 roundings of at most U in sequence. The interval so
+// bounded straddles a rounding boundary of the float for about one row in
+// 10^4 to 10^3 (26,000 to 262,144 fine terms); those are replayed. Before,
+// every row whose terms span more than 53 bits was (sigma-3 logits,
+// V = 262,144): 48 bf16 rows of which 8 are full order 324 -> 151 us a call, one
+// f32 row 245 -> 203 us, 64 f32 rows 828 -> 634 us.
+__device__ __forceinline__ bool den_rounds_alike(double S, uint32_t fine, int V) {
+    if (!(S >= 0.5) || !(S < 0x1p60)) return false;
+    const double eps = (static_cast<double>(fine) + 64.0 + 2.0 * (static_cast<double>(V) / 512.0 + 512.0)) *
+                       __builtin_ldexp(1.0, sum_exp(S) - 53) * (1.0 + 0x1p-10);
+    return static_cast<float>(1.0 / (S - eps)) == static_cast<float>(1.0 / (S + eps));
+}
+
+// How far two double sums of `n` probabilities in different orders, and of one
+// term more, can lie apart (the sums are below 2: at most 2^-53 a rounding).
+__device__ __forceinline__ double near_sum_error(uint32_t n) { return (2.0 * n + 16.0) * 0x1p-53 * (1.0 + 0x1p-10); }
+
+// Whether |x - c| < 1e-6 is decided for every c within eps of `c`; `near` is
+// its value then.
+__device__ __forceinline__ bool near_decided(double x, double c, double eps, bool& near) {
+    const double d = __builtin_fabs(x - c);
+    near = d < 1e-6;
+    return d <= 1e-6 - eps || d >= 1e-6 + eps;
+}
+
 // Whether a sorted row's denominator needs no replay: its certificate (the
 // parallel sum S, the lowest set bit of every term, NaN) from the meta words
 // (a NaN term makes the sum NaN: no replay either).
-__device__ __forceinline__ bool den_certified(const uint32_t* meta, double& S) {
+__device__ __forceinline__ bool den_certified(const uint32_t* meta, double& S, uint32_t k, int V) {
     S = __builtin_bit_cast(double, (static_cast<uint64_t>(meta[kMetaSumHi]) << 32) | meta[kMetaSumLo]);
     const int minlsb = static_cast<int>(meta[kMetaMinLsb]);
     const bool nan = meta[kMetaAnyNan] != 0u;
-    return nan || S == 0.0 || minlsb >= exp_of(S) - 51;
+    return nan || S == 0.0 || minlsb >= exp_of(S) - 51 || den_rounds_alike(S, k, V);
 }
 
 // The largest binade the sequential sum can reach: that of the parallel sum
@@ -1779,7 +1816,7 @@ __device__ __forceinline__ bool map_part_needed(const DevArgs& a, int row, int p
     if (meta[kMetaStatus] != (a.fo_fallback ? kStatusFallback : kStatusOk)) return false;
     if (part * kMapSubItems >= static_cast<int>(meta[kMetaItems])) return false;
     double S;
-    return !den_certified(meta, S);
+    return !den_certified(meta, S, k, a.vocab);
 }
 
 // The maps of one part (block-uniform): its items' elements in [1, k)
@@ -1797,7 +1834,7 @@ __device__ __forceinline__ void map_part(const DevArgs& a, int row, int part, ui
     const uint32_t* meta = a.fo_meta + static_cast<int64_t>(row) * kMetaWords;
     const int G = static_cast<int>(meta[kMetaItems]);
     double S;
-    (void)den_certified(meta, S);
+    (void)den_certified(meta, S, k, V);
     const int i0 = part * kMapSubItems;
     const uint32_t* pre = a.fo_pre + static_cast<int64_t>(row) * a.fo_items_stride;
     const float* aux = a.fo_aux + static_cast<int64_t>(row) * a.fo_items_stride;
@@ -2159,8 +2196,9 @@ __global__ __launch_bounds__(kDThreads, kSorted ? 2 : 4) void fo_decide_kernel(D
     // Every term is a multiple of 2^minlsb; if the sum needs at most 53 bits
     // above that, every partial sum in every order is exact, so the parallel
     // sum equals the reference's sequential one (generation.cpp:97).
-    const bool certified = !any_nan && (Sp == 0.0 || ml >= exp_of(Sp) - 51);
+    bool certified = !any_nan && (Sp == 0.0 || ml >= exp_of(Sp) - 51);
     if constexpr (kSorted) {
+        if (!any_nan && !certified) certified = den_rounds_alike(Sp, k, V);
         // up to V single-token items: the whole block replays the sum
         double den = Sp;
         if (any_nan) {
@@ -2176,7 +2214,21 @@ __global__ __launch_bounds__(kDThreads, kSorted ? 2 : 4) void fo_decide_kernel(D
             den = s2;
         }
         if (tid == 0) sh.den = den;
-    } else if (wave == 0) {
+    } else {
+        if (!any_nan && !certified) {  // (block-uniform) terms that may round when added
+            const float tiny = __builtin_ldexpf(1.0f, min(sum_exp(Sp) - 29, 0));
+            uint32_t fine = 0;
+            for (int i = tid; i < G; i += kDThreads) {  // this thread staged item i in 4a
+                const float pe = i < kStage ? sh.st.add[i] : aux[i];
+                const uint32_t st = i <= kStage ? sh.st.pre[i] : pre[i];
+                if (pe < tiny) fine += top_k_count(st, static_cast<uint32_t>(items[i]), k);
+            }
+            uint32_t all;
+            (void)dblock_excl_scan(fine, sh.scan, all);
+            certified = den_rounds_alike(Sp, all, V);
+        }
+    }
+    if (!kSorted && wave == 0) {
         double den = Sp;
         if (any_nan) {
             den = __builtin_nan("");
@@ -2318,7 +2370,12 @@ __global__ __launch_bounds__(kDThreads, kSorted ? 2 : 4) void fo_decide_kernel(D
                 }
                 sum = wave_reduce(sum, [](double x, double y) { return x + y; });
                 mlb = wave_reduce(mlb, [](int x, int y) { return min(x, y); });
-                if (sum == 0.0 || mlb >= exp_of(sum) - 51) {
+                // or one that no order of the sum would decide otherwise
+                const double eps = near_sum_error(pos);
+                const double c = static_cast<double>(choice);
+                bool nb, na;
+                if (sum == 0.0 || mlb >= exp_of(sum) - 51 ||
+                    (near_decided(c, sum, eps, nb) && near_decided(c, sum + static_cast<double>(iv.addend(item)), eps, na))) {
                     c_before = sum;
                 } else {
                     ChainPos cp2{0, 1};
@@ -2772,7 +2829,11 @@ __global__ __launch_bounds__(kDThreads, kSorted ? 2 : 4) void fo_decide_kernel(D
                     sum += sh.dred[w];
                     mlb = min(mlb, sh.ired[w]);
                 }
-                if (sum == 0.0 || mlb >= exp_of(sum) - 51) {
+                const double eps = near_sum_error(d.pos);
+                const double c = static_cast<double>(choice);
+                bool nb, na;
+                if (sum == 0.0 || mlb >= exp_of(sum) - 51 ||
+                    (near_decided(c, sum, eps, nb) && near_decided(c, sum + static_cast<double>(aux[d.item] * inv), eps, na))) {
                     c_before = sum;
                 } else {
                     ChainPos cp2{0, 1};
