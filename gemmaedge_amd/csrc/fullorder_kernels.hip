@@ -41,6 +41,7 @@
 #include "chain_block.h"
 #include "chain_math.h"
 #include "chain_wave.h"
+#include "fullorder_common.h"
 #include "ge_math.h"
 #include "sampler_internal.h"
 
@@ -59,16 +60,6 @@ constexpr uint32_t kLowBin = 0x007Fu;     // -inf
 constexpr uint32_t kHighBin = 0xFF80u;    // +inf
 constexpr int kSpillCap = 512;
 constexpr uint64_t kSat = static_cast<uint64_t>(1) << 62;
-
-enum : uint32_t {
-    kMetaItems = 0, kMetaExtras = 1, kMetaNan = 2, kMetaStatus = 3,
-    // sorted rows only: the top k's exps, from the sort kernel (their sum
-    // as two words of a double, the lowest set bit, any NaN)
-    kMetaSumLo = 4, kMetaSumHi = 5, kMetaMinLsb = 6, kMetaAnyNan = 7
-};
-// kStatusFallback: items of a flagged bf16 row, made by the fallback sort;
-// kStatusSkip: a row the fallback pass leaves as the first pass wrote it.
-enum : uint32_t { kStatusOk = 0, kStatusTooManyPenalised = 1, kStatusFallback = 2, kStatusSkip = 3 };
 
 // ---- bf16 order-key bins ---------------------------------------------------
 
@@ -93,26 +84,6 @@ __device__ __forceinline__ float load_value(const uint16_t* rowp, int i) { retur
 
 __device__ __forceinline__ ge_sample_params params_of(const DevArgs& a, int row) {
     return a.row_params ? a.row_params[row] : a.params;
-}
-
-// generation.cpp:66, :80 — rows this path serves: sampling (T > 0 or NaN) with k > kMaxTopK.
-__device__ __forceinline__ bool full_order_row(const ge_sample_params& p, int V, uint32_t& k) {
-    if (p.temperature <= 0.0f) return false;
-    k = p.top_k ? min(p.top_k, static_cast<uint32_t>(V)) : static_cast<uint32_t>(V);
-    return k > static_cast<uint32_t>(kMaxTopK);
-}
-
-__device__ __forceinline__ void history_of(const DevArgs& a, int row, const int32_t*& h, int& n) {
-    h = nullptr;
-    n = 0;
-    if (a.ring) {
-        h = a.ring + static_cast<int64_t>(row) * a.ring_capacity;
-        n = min(max(a.ring_len[row], 0), a.ring_capacity);
-    } else if (a.history && a.history_offsets) {
-        const int s = a.history_offsets[row];
-        h = a.history + s;
-        n = max(a.history_offsets[row + 1] - s, 0);
-    }
 }
 
 __device__ __forceinline__ uint32_t rl32(uint32_t v, int lane) {
@@ -221,10 +192,6 @@ __device__ __forceinline__ int lsb_exp(float x) {  // exponent of the lowest set
     const uint32_t man = b & 0x7fffffu;
     if (ex == 0) return -149 + __builtin_ctz(man);
     return static_cast<int>(ex) - 150 + __builtin_ctz(man | 0x800000u);
-}
-
-__device__ __forceinline__ int exp_of(double d) {  // floor(log2 d), d > 0 normal
-    return static_cast<int>((__builtin_bit_cast(uint64_t, d) >> 52) & 0x7ff) - 1023;
 }
 
 // ---- kernel 1: histogram and item list --------------------------------------
@@ -418,7 +385,7 @@ __global__ __launch_bounds__(kThreads) void fo_hist_kernel(DevArgs a) {
             meta[kMetaItems] = 0;
             meta[kMetaExtras] = 0;
             meta[kMetaNan] = 0;
-            meta[kMetaStatus] = kStatusTooManyPenalised;
+            meta[kMetaStatus] = kStatusToSort;
         }
         return;
     }
@@ -665,13 +632,6 @@ struct SortShared {
     uint32_t ured[kWaves];
 };
 
-// Buffer reads of the sort read from L2 (agent-scope loads skip the CU's L1),
-// so a line the L1 kept from an earlier pass is never used after another wave
-// of the workgroup rewrote it; the writers wait for their stores before each
-// barrier.
-__device__ __forceinline__ uint32_t ld_l2(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ __forceinline__ void stores_done_barrier() {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -717,7 +677,7 @@ __global__ __launch_bounds__(kThreads) void fo_sort_kernel(DevArgs a) {
         // row); the decide kernel of this pass skips the others.
         const uint32_t st = a.fo_meta[static_cast<int64_t>(a.fo_row0 + row) * kMetaWords + kMetaStatus];
         __syncthreads();  // every thread has read it before thread 0 may rewrite it below
-        if (st != kStatusTooManyPenalised) {
+        if (st != kStatusToSort) {
             if (tid == 0) a.fo_meta[static_cast<int64_t>(row) * kMetaWords + kMetaStatus] = kStatusSkip;
             return;
         }
@@ -1756,43 +1716,6 @@ __host__ __device__ constexpr int64_t map_row_words(int vocab) {
     return static_cast<int64_t>((vocab + kMapTile - 1) / kMapTile) * kMapSub * kMapPartWords;
 }
 
-// The exponent whose binade holds the sequential sum that S approximates (the
-// two differ by far less than 2^-20), or the one above.
-__device__ __forceinline__ int sum_exp(double S) { return exp_of(S * (1.0 + 0x1p-20)); }
-
-// Whether the reciprocal 1 / den rounds to the same float for every value that
-// the reference's sequential double sum can have, S being a sum of the same
-// terms in another order: then no replay is needed, as only that float is
-// used (generation.cpp:98-101). With e = sum_exp(S) and U = 2^(e-52), a term
-// whose lowest set bit is at least U adds without rounding except where the
-// sum enters a higher binade (the sum starts at exp(0) = 1, so at most e
-// times); a float at or above 2^(e-29) is such a term. Each other term
-// (`fine` of them, or more) rounds by at most U / 2. The parallel sum adds at
-// most V / 512 + 512 roundings of at most U in sequence. The interval so
-// bounded straddles a rounding boundary of the float for about one row in
-// 10^4 to 10^3 (26,000 to 262,144 fine terms); those are replayed. Before,
-// every row whose terms span more than 53 bits was (sigma-3 logits,
-// V = 262,144): 48 bf16 rows of which 8 are full order 324 -> 151 us a call, one
-// f32 row 245 -> 203 us, 64 f32 rows 828 -> 634 us.
-__device__ __forceinline__ bool den_rounds_alike(double S, uint32_t fine, int V) {
-    if (!(S >= 0.5) || !(S < 0x1p60)) return false;
-    const double eps = (static_cast<double>(fine) + 64.0 + 2.0 * (static_cast<double>(V) / 512.0 + 512.0)) *
-                       __builtin_ldexp(1.0, sum_exp(S) - 53) * (1.0 + 0x1p-10);
-    return static_cast<float>(1.0 / (S - eps)) == static_cast<float>(1.0 / (S + eps));
-}
-
-// How far two double sums of `n` probabilities in different orders, and of one
-// term more, can lie apart (the sums are below 2: at most 2^-53 a rounding).
-__device__ __forceinline__ double near_sum_error(uint32_t n) { return (2.0 * n + 16.0) * 0x1p-53 * (1.0 + 0x1p-10); }
-
-// Whether |x - c| < 1e-6 is decided for every c within eps of `c`; `near` is
-// its value then.
-__device__ __forceinline__ bool near_decided(double x, double c, double eps, bool& near) {
-    const double d = __builtin_fabs(x - c);
-    near = d < 1e-6;
-    return d <= 1e-6 - eps || d >= 1e-6 + eps;
-}
-
 // Whether a sorted row's denominator needs no replay: its certificate (the
 // parallel sum S, the lowest set bit of every term, NaN) from the meta words
 // (a NaN term makes the sum NaN: no replay either).
@@ -2026,23 +1949,6 @@ __device__ __forceinline__ uint32_t dblock_excl_scan(uint32_t v, uint32_t* scrat
     }
     __syncthreads();
     return before + incl - v;
-}
-
-// First index in [lo, hi) whose predicate is false, for a predicate that is
-// true on a prefix; 64-way search with one wave.
-template <typename Pred>
-__device__ uint32_t wave_partition_point(uint32_t lo, uint32_t hi, Pred pred) {
-    const int lane = __lane_id();
-    while (hi > lo) {
-        const uint32_t step = (hi - lo + 63) / 64;
-        const uint32_t probe = lo + static_cast<uint32_t>(lane) * step;
-        const uint64_t m = __ballot(probe < hi && pred(probe));
-        if (m == 0) break;  // pred(lo) is false
-        const int last = 63 - static_cast<int>(__builtin_clzll(m));
-        lo = lo + static_cast<uint32_t>(last) * step + 1;
-        hi = min(hi, lo - 1 + step);
-    }
-    return lo;
 }
 
 // The same partition point, searched first in the 64 keys from w0 = c - 32
@@ -3235,7 +3141,32 @@ template <typename T>
 hipError_t sorted_pass(const DevArgs& a, hipStream_t stream) {
     const int64_t stride = fo_items_stride_f32(a.vocab);
     if (a.fo_capacity < stride) return hipErrorInvalidValue;
-    const int64_t per64 = std::min<int64_t>(a.fo_capacity / stride, a.rows);
+    int64_t per64 = std::min<int64_t>(a.fo_capacity / stride, a.rows);
+    // f32 rows with k = V need no sort (fullorder_binned.hip); the sort-based
+    // kernels then serve the rows it leaves. Shared parameters with
+    // 1024 < top_k < V go to them straight away, and calls with per-row
+    // parameters: the host cannot tell whether any row needs this path, and its
+    // launches cost 20 us when every row leaves at once.
+    const bool binned = std::is_same<T, float>::value && !a.fo_fallback && a.fo_tiles != nullptr && !a.row_params &&
+                        (a.params.top_k == 0u || a.params.top_k >= static_cast<uint32_t>(a.vocab)) &&
+                        a.fo_tiles_words >= fb_row_words(a.vocab);
+    if (binned) {
+        per64 = std::min(per64, a.fo_tiles_words / fb_row_words(a.vocab));
+        for (int r0 = 0; r0 < a.rows; r0 += static_cast<int>(per64)) {
+            DevArgs s = slice_rows(a, r0, static_cast<int>(std::min<int64_t>(per64, a.rows - r0)));
+            s.fo_items_stride = stride;
+            s.fo_row0 = 0;  // (the fallback reads the status of this slice's workspace rows)
+            hipError_t e = launch_binned(s, stream);
+            if (e != hipSuccess) return e;
+            s.fo_fallback = 1;
+            s.fo_maps = 0;
+            hipLaunchKernelGGL(fo_sort_kernel<T>, dim3(s.rows), dim3(kThreads), 0, stream, s);
+            hipLaunchKernelGGL((fo_decide_kernel<T, true>), dim3(s.rows), dim3(kDThreads), 0, stream, s);
+            e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     // f32 slices of up to kSplitMaxRows rows take the many-workgroup sort
     // (when the handle's tile area holds them): its time grows with the rows,
     // while fo_sort_kernel runs up to 256 rows side by side in about the time

@@ -161,8 +161,9 @@ int ge_sampler_create(int device, int max_rows, int max_vocab, int max_history, 
         alloc(reinterpret_cast<void**>(&s->fo_extras), rows * static_cast<size_t>(s->fo_extras_cap) * sizeof(uint64_t));
         alloc(reinterpret_cast<void**>(&s->fo_bitmap), words * sizeof(uint32_t));
         alloc(reinterpret_cast<void**>(&s->fo_meta), rows * ge::kMetaWords * sizeof(uint32_t));
-        // the many-workgroup f32 sort: per-tile counts for the same 256 rows
-        s->fo_tiles_words = static_cast<int64_t>(f32_rows) * ge::fo_tile_words(ge::fo_split_tiles(max_vocab));
+        // the same 256 rows' per-tile counts (many-workgroup sort) or bins
+        s->fo_tiles_words = static_cast<int64_t>(f32_rows) *
+                            std::max(ge::fo_tile_words(ge::fo_split_tiles(max_vocab)), ge::fb_row_words(max_vocab));
         alloc(reinterpret_cast<void**>(&s->fo_tiles), static_cast<size_t>(s->fo_tiles_words) * sizeof(uint32_t));
         if (e == hipSuccess) e = hipMemset(s->fo_bitmap, 0, words * sizeof(uint32_t));
     }

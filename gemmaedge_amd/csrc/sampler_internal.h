@@ -79,7 +79,7 @@ struct DevArgs {
     int32_t fo_extras_cap;        // <= kFoExtrasCap
     int64_t fo_bitmap_words;
     int64_t fo_capacity;          // items (and aux, pre entries) in the workspace
-    uint32_t* fo_tiles;           // [fo_tiles_words] f32 rows' per-tile counts and partials (many-workgroup sort)
+    uint32_t* fo_tiles;           // [fo_tiles_words] f32 rows' per-tile counts (many-workgroup sort) or bins (no sort)
     int64_t fo_tiles_words;
     // Full-order fallback pass (bf16 rows with more unique penalised ids than
     // fo_extras_cap): the sort-based kernels serve only the rows the first
@@ -109,6 +109,18 @@ inline int64_t fo_items_stride_f32(int vocab) { return (static_cast<int64_t>(voc
 // 256 digit counts, an item count and four partial words.
 constexpr int fo_split_tiles(int vocab) { return (vocab + 4095) / 4096; }
 constexpr int64_t fo_tile_words(int tiles) { return static_cast<int64_t>(tiles) * (256 + 1 + 4); }
+
+// f32 rows without a sort (fullorder_binned.hip): histogram bins per row (about
+// one per 16 tokens), and the words of a row's area in fo_tiles.
+constexpr int kFbMaxBins = 16384;
+constexpr int kFbParts = 64;    // workgroups that stream one row, at most
+constexpr int kFbSegs = 4096;   // expanded bins of one row, at most
+__host__ __device__ constexpr int fb_bins(int vocab) {
+    return vocab >= 131072 ? kFbMaxBins : vocab >= 65536 ? kFbMaxBins / 2 : vocab >= 32768 ? kFbMaxBins / 4 : kFbMaxBins / 8;
+}
+__host__ __device__ constexpr int64_t fb_row_words(int vocab) {
+    return fb_bins(vocab) + 6 * kFbParts + 64 + kFbMaxBins / 32 + 3 * kFbSegs;
+}
 
 // The row's parameters: the shared ones, or its entry of row_params.
 __device__ __forceinline__ ge_sample_params row_params(const DevArgs& a, int row) {
@@ -186,6 +198,11 @@ hipError_t launch_stream(const DevArgs& a, hipStream_t stream);
 // Launches the greedy kernel (every row greedy, shared parameters): one pass,
 // ept in {16, 64}. Returns a hipError_t.
 hipError_t launch_greedy(const DevArgs& a, hipStream_t stream, int ept);
+
+// Launches the sort-free full-order kernels on rows [0, a.rows) (f32, a slice
+// that the workspace holds: a.fo_items_stride = fo_items_stride_f32(vocab));
+// rows it does not serve get the meta status kStatusToSort.
+hipError_t launch_binned(const DevArgs& a, hipStream_t stream);
 
 // Launches the full-order kernels (rows with k > kMaxTopK; other rows are
 // skipped): one pair for bf16, one pair per slice of rows for f32. Returns a
