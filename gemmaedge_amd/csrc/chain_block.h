@@ -165,14 +165,9 @@ __device__ __forceinline__ bool exceeds(const Bin& b, U r) {
 // Returns true on a stop with cp at the stop element; otherwise false with
 // cp.elem == L and cp.item holding element L - 1. Requires L <= start(G);
 // pre and add 16-byte aligned. Item i's addend is add[i] * scale.
-// `log(item, s)` is called by every thread after each event (the item that left
-// the binade or reached the threshold), with the accumulator after it.
-struct NoLog {
-    __device__ void operator()(int, double) {}
-};
-template <typename A, bool kDesc, int kThreads, typename Log>
+template <typename A, bool kDesc, int kThreads>
 __device__ bool block_chain(const uint32_t* pre_p, const float* add_p, float scale, int G, ChainPos& cp_io, uint32_t L,
-                            double& s_io, double thr, Shared<kThreads / 64>& sh_p, Log& log) {
+                            double& s_io, double thr, Shared<kThreads / 64>& sh_p) {
     ChainPos cp = cp_io;  // (locals: the references may be memory of the caller's)
     double s = s_io;
     auto leave = [&](bool r) {
@@ -250,7 +245,6 @@ __device__ bool block_chain(const uint32_t* pre_p, const float* add_p, float sca
                     cp.elem = sh.prelem[pbuf];
                     const bool hit = sh.prhit[pbuf] != 0;
                     pbuf ^= 1;
-                    log(pe, s);
                     if (hit || cp.elem >= L) {
                         cp.item = pe;
                         return leave(hit);
@@ -363,7 +357,6 @@ __device__ bool block_chain(const uint32_t* pre_p, const float* add_p, float sca
             s = sh.rs;
             cp.elem = sh.relem;
             const bool hit = sh.rhit != 0;
-            log(fe, s);
             if (hit || cp.elem >= L) {
                 cp.item = fe;
                 return leave(hit);
@@ -377,13 +370,6 @@ __device__ bool block_chain(const uint32_t* pre_p, const float* add_p, float sca
 #pragma unroll
         for (int j = 0; j < kPer; ++j) ab[j] = nab[j];
     }
-}
-
-template <typename A, bool kDesc, int kThreads>
-__device__ __forceinline__ bool block_chain(const uint32_t* pre, const float* add, float scale, int G, ChainPos& cp,
-                                            uint32_t L, double& s, double thr, Shared<kThreads / 64>& sh) {
-    NoLog none;
-    return block_chain<A, kDesc, kThreads, NoLog>(pre, add, scale, G, cp, L, s, thr, sh, none);
 }
 
 }  // namespace bchain

@@ -6,38 +6,42 @@
 // binade of the accumulator such a sum moves by whole ulps, and the number of
 // ulps that an addend q adds, round(q / ulp), does not depend on the order
 // (chain_math.h; an exact tie does, through the accumulator's parity). So the
-// order only matters where the accumulator changes binade, where an addend ties,
-// and where the sum stops. Everywhere else a run of neighbouring addends that
-// all round to the same number of ulps is one item (count, any of the
-// addends) of the closed-form chain. A row of V = 262,144 near-uniform
-// logits then has some 25,000 items in place of 262,144 sorted tokens, and a
-// confident row a few thousand.
+// order only matters where the accumulator changes binade, where an addend
+// ties, and where the sum stops. The row is therefore cut into bins of
+// neighbouring probabilities: where all of a bin's addends round alike it is a
+// count times an integer, where they do not its tokens' integers are summed,
+// and only the bins with a binade change, a tie or a stop (a few thousand
+// tokens of a near-uniform row of V = 262,144) are sorted and taken one by one.
 //
 //   fb_range    marks the history ids; the row's largest final value and
 //               smallest raw one
 //   fb_exps     every token's exp((v - max) / T), kept; their sum; their
 //               histogram in bins of equal width in the float's bits
 //   fb_plan     1 / denominator; per bin the probabilities' sum before it and
-//               the walk's, following the float sums' rounding; which bins
-//               must be expanded into single tokens (a binade change, the
-//               top-p, min-p or draw stop, or not all addends alike there)
+//               the walk's, following the float sums' rounding; the ulps of the
+//               bins whose addends round alike; which bins are expanded into
+//               tokens, and which of those the chains replay
 //   fb_collect  the expanded bins' tokens; the sum of the probabilities
 //               before the bins the draw can end in
-//   fb_order    the expanded bins' tokens in order
-//   fb_draw     the chains over the items, the token, and a check that every
-//               unexpanded bin was passed in the binade the plan assumed
+//   fb_order    the expanded bins' ulps, or their tokens in order
+//   fb_draw     the chains, the token, and a check that the bins between two
+//               replayed ones were passed in the binade the plan took them in
 //
 // Results are exact for any plan: fb_draw checks what the plan assumed
 // and otherwise leaves the row to the sort-based pass, as do rows that this
 // path does not serve (NaN or infinite maxima, a denominator whose
-// reciprocal the sum's error interval leaves open, expanded bins of more than
+// reciprocal the sum's error interval leaves open, replayed bins of more than
 // kFbSegMost tokens).
+//
+// Measured against the radix sort it replaces (whole calls, V = 262,144): one
+// row 245 -> 106 us, 64 rows 824 -> 216 us, 512 near-uniform rows 4,822 ->
+// 1,281 us; of the last, per 256 rows: range 63, exps 237, plan 55, collect 92,
+// order 105, draw 87 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <climits>
 
-#include "chain_block.h"
 #include "chain_math.h"
 #include "fullorder_common.h"
 #include "ge_math.h"
@@ -57,8 +61,26 @@ constexpr uint32_t kLeast = 0x2f800000u;  // 2^-32: smaller exps share the last 
 constexpr uint32_t kFbHead = 1024;     // tokens always expanded
 constexpr int kFbWaveSeg = 512;        // tokens of a bin that one wave orders
 constexpr uint32_t kFbSegMost = 4096;  // tokens of an expanded bin at most
-constexpr double kFbDrift = 0x1p-11;   // the plan's relative margin on a float sum
-constexpr uint64_t kFbRegular = 1ull << 63;  // an item that stands for a whole bin
+constexpr double kFbDrift = 0x1p-13;   // the plan's relative margin on a float sum
+
+// One expanded bin. What the chains add (cumulative) or take off (walk) for the
+// bins between two replayed ones is a sum of whole ulps of one binade.
+struct FbSeg {
+    uint32_t item;    // its tokens' first item
+    uint32_t n;       // its tokens
+    uint32_t elem;    // its first element (the tokens before it)
+    uint32_t info;    // biased exponents of the two accumulators before it, and kSeg* flags
+    double cum;       // ulps that the unexpanded bins before it add to the cumulative
+    double walk;      // ulps that they take off in the walk
+    uint32_t scum;    // ulps that this bin's own tokens add, when it is not replayed
+    uint32_t swalk;
+};
+static_assert(sizeof(FbSeg) == 4 * kFbSegWords, "the area's size");
+enum : uint32_t {
+    kSegReplayCum = 1u << 16,   // the cumulative takes its tokens one by one
+    kSegReplayWalk = 1u << 17,  // the walk does
+    kSegInWalk = 1u << 18       // the walk may reach it
+};
 
 // The row's area in fo_tiles.
 struct FbRow {
@@ -69,9 +91,9 @@ struct FbRow {
     double* pbef;     // [kFbParts] sums of the probabilities before the draw's bins
     uint32_t* scal;   // [kScalWords]
     uint32_t* mask;   // [bins / 32] expanded bins
-    uint32_t* seg;    // [3 * kFbSegs] item, tokens and first element of each expanded bin
+    FbSeg* seg;       // [kFbSegs + 1] the expanded bins, in order, and the list's end
 };
-enum : int { kScShift = 0, kScInv, kScDrawBin, kScDrawItem, kScDrawEnd, kScSegs, kScalWords = 64 };
+enum : int { kScShift = 0, kScInv, kScDrawBin, kScDrawItem, kScDrawEnd, kScSegs, kScCut, kScalWords = 64 };
 
 __device__ __forceinline__ FbRow fb_row(const DevArgs& a, int row, int bins) {
     uint32_t* w = a.fo_tiles + static_cast<int64_t>(row) * fb_row_words(a.vocab);
@@ -83,7 +105,7 @@ __device__ __forceinline__ FbRow fb_row(const DevArgs& a, int row, int bins) {
     r.pbef = r.psum + kFbParts;
     r.scal = reinterpret_cast<uint32_t*>(r.pbef + kFbParts);
     r.mask = r.scal + kScalWords;
-    r.seg = r.mask + kFbMaxBins / 32;
+    r.seg = reinterpret_cast<FbSeg*>(r.mask + kFbMaxBins / 32);
     return r;
 }
 // The row's exps, in the upper half of its items (fb_half() items are left).
@@ -148,9 +170,12 @@ __device__ __forceinline__ uint32_t fb_block_max(uint32_t v, uint32_t* s) {
 
 // 1. The part's history bits, its largest final key and smallest raw key.
 //    A streaming read: bound by memory at many rows, by latency at few.
-__global__ __launch_bounds__(kFT) void fb_range_kernel(DevArgs a) {
-    __shared__ uint32_t s[kFW];
-    const int row = blockIdx.y, part = blockIdx.x, parts = gridDim.x, tid = threadIdx.x;
+struct RangeShared {
+    uint32_t s[kFW];
+};
+__device__ __forceinline__ void fb_range(const DevArgs& a, int row, int part, int parts, RangeShared& sh) {
+    uint32_t* s = sh.s;
+    const int tid = threadIdx.x;
     ge_sample_params p;
     const int bins = fb_bins(a.vocab);
     if (!fb_serves(a, row, p)) {
@@ -222,31 +247,36 @@ __device__ __forceinline__ void fb_bin_shape(const FbRow& r, int parts, int bins
 //    capped and penalised value), the part's sum of them, and the histogram of
 //    their bins. Bound by the exact tanhf and expf (about 130 instructions a
 //    token), which a step's 16 tokens per thread overlap.
-__global__ __launch_bounds__(kFT) void fb_exps_kernel(DevArgs a) {
-    __shared__ uint32_t hist_s[kFbMaxBins];
-    __shared__ uint64_t tab[32];
-    __shared__ double sums[kFW];
-    __shared__ float s_vmax;
-    __shared__ uint32_t s_shift;
-    const int row = blockIdx.y, part = blockIdx.x, parts = gridDim.x, tid = threadIdx.x;
+struct ExpsShared {
+    uint32_t hist[kFbMaxBins];
+    uint64_t tab[32];
+    double sums[kFW];
+    float vmax;
+    uint32_t shift;
+};
+__device__ __forceinline__ void fb_exps(const DevArgs& a, int row, int part, int parts, ExpsShared& sh) {
+    uint32_t* hist_s = sh.hist;
+    uint64_t* tab = sh.tab;
+    double* sums = sh.sums;
+    const int tid = threadIdx.x;
     ge_sample_params p;
     if (!fb_serves(a, row, p)) return;
     const int bins = fb_bins(a.vocab);
     const FbRow r = fb_row(a, row, bins);
     if (tid < 64) {
         float vm;
-        uint32_t sh;
-        fb_bin_shape(r, parts, bins, p, vm, sh);
+        uint32_t sf;
+        fb_bin_shape(r, parts, bins, p, vm, sf);
         if (tid == 0) {
-            s_vmax = vm;
-            s_shift = sh;
+            sh.vmax = vm;
+            sh.shift = sf;
         }
         if (tid < 32) tab[tid] = exp2_table(static_cast<uint32_t>(tid));
     }
     for (int i = tid; i < bins; i += kFT) hist_s[i] = 0u;
     __syncthreads();
-    const float vmax = s_vmax;
-    const uint32_t shift = s_shift;
+    const float vmax = sh.vmax;
+    const uint32_t shift = sh.shift;
     int lo, hi;
     fb_part(a, part, parts, lo, hi);
     const int32_t* hist;
@@ -303,6 +333,7 @@ __global__ __launch_bounds__(kFT) void fb_exps_kernel(DevArgs a) {
 
 // Exclusive prefix of one double (count) per thread over the workgroup, and
 // the total. The order of the additions is fixed.
+template <int kWaves>
 __device__ __forceinline__ double fb_scan_f64(double v, double* s, double& total) {
     const int wave = threadIdx.x >> 6;
     const double incl = wave::incl_f64(v);
@@ -310,13 +341,14 @@ __device__ __forceinline__ double fb_scan_f64(double v, double* s, double& total
     __syncthreads();
     double before = 0.0;
     total = 0.0;
-    for (int w = 0; w < kFW; ++w) {
+    for (int w = 0; w < kWaves; ++w) {
         if (w == wave) before = total;
         total += s[w];
     }
     __syncthreads();
     return before + (incl - v);
 }
+template <int kWaves>
 __device__ __forceinline__ uint32_t fb_scan_u32(uint32_t v, uint32_t* s, uint32_t& total) {
     const int wave = threadIdx.x >> 6;
     const uint32_t incl = wave::incl_add(v);
@@ -324,7 +356,7 @@ __device__ __forceinline__ uint32_t fb_scan_u32(uint32_t v, uint32_t* s, uint32_
     __syncthreads();
     uint32_t before = 0;
     total = 0;
-    for (int w = 0; w < kFW; ++w) {
+    for (int w = 0; w < kWaves; ++w) {
         if (w == wave) before = total;
         total += s[w];
     }
@@ -335,72 +367,97 @@ __device__ __forceinline__ uint32_t fb_scan_u32(uint32_t v, uint32_t* s, uint32_
 // The biased float exponent of x > 0, at least 1 (subnormal floats share the
 // first normal binade's ulp); 0 for x <= 0.
 __device__ __forceinline__ int fb_expo(double x) {
-    if (!(x > 0.0)) return 0;
-    return max(static_cast<int>((__builtin_bit_cast(uint64_t, x) >> 52) & 0x7ff) - 1023 + 127, 1);
+    const int e = static_cast<int>(__builtin_bit_cast(uint64_t, x) >> 52) - 1023 + 127;
+    return x > 0.0 ? max(e, 1) : 0;
 }
-// 1 / ulp of the float binade with biased exponent e.
-__device__ __forceinline__ double fb_inv_ulp(int e) { return __builtin_ldexp(1.0, 150 - e); }
-// Whether every addend of [lo, hi] adds the same whole number of ulps in the
-// binade, none of them a tie.
-__device__ __forceinline__ bool fb_alike(float lo, float hi, int e) {
-    const double iu = fb_inv_ulp(e);
-    const double yl = static_cast<double>(lo) * iu, yh = static_cast<double>(hi) * iu;  // exact
-    const double n = __builtin_floor(yh + 0.5);
-    return yh < 0x1p24 && yl > n - 0.5 && yh < n + 0.5;
+// Whether every addend of [lo, hi] adds the same whole number `n` of ulps in
+// the binade with biased exponent e (ulp 2^(e - 150)), none of them a tie.
+// (Scaling by a power of two and, below 2^22, adding 1/2 are exact.)
+__device__ __forceinline__ bool fb_alike(float lo, float hi, int e, uint32_t& n) {
+    const float yl = __builtin_ldexpf(lo, 150 - e), yh = __builtin_ldexpf(hi, 150 - e);
+    const float f = __builtin_floorf(yh + 0.5f);
+    const bool ok = yh < 0x1p22f && yl > f - 0.5f && yh < f + 0.5f;
+    n = ok ? static_cast<uint32_t>(f) : 0u;
+    return ok;
 }
 
-// 3. One workgroup per row; thread t holds bins kPer * t .. Latency-bound: five
-//    workgroup scans.
+// 3. One workgroup per row; thread t holds bins kPer * t .., which stay in LDS
+//    (kept in registers, 16 bins a thread spill: one row 88 us instead of 36).
+//    Bound by its sweeps over the bins on one CU.
+struct PlanShared {
+    uint32_t c[kFbMaxBins + kFbMaxBins / 16];  // counts (padded: a thread's bins lie 17 words from the next's)
+    uint32_t w[kFbMaxBins + kFbMaxBins / 16];  // the bin's rounded sum (a float), then what it is
+    double sd[kFW];
+    uint32_t su[kFW];
+    uint32_t mask[kFbMaxBins / 32];
+    uint32_t bad, cut, stop, first, last, off0, off1;
+    double cut_lo, cut_hi;
+    float stop_q;
+};
 template <int kPer>
-__global__ __launch_bounds__(kFT) void fb_plan_kernel(DevArgs a, int parts) {
-    __shared__ double sd[kFW];
-    __shared__ uint32_t su[kFW];
-    __shared__ uint32_t smask[kFbMaxBins / 32];
-    __shared__ uint32_t s_bad, s_cut, s_stop, s_first, s_last, s_off0, s_off1;
-    __shared__ double s_cut_lo, s_cut_hi;
-    __shared__ float s_stop_q;
+__device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, PlanShared& sh) {
     constexpr int kBins = kPer * kFT;
-    const int row = blockIdx.x, tid = threadIdx.x, lane = __lane_id();
+    const int tid = threadIdx.x, lane = __lane_id();
     ge_sample_params p;
     if (!fb_serves(a, row, p)) return;
     const int V = a.vocab;
     const FbRow r = fb_row(a, row, kBins);
     uint32_t* meta = fb_meta(a, row);
-    uint32_t* pre = a.fo_pre + static_cast<int64_t>(row) * a.fo_items_stride;
-    float* aux = a.fo_aux + static_cast<int64_t>(row) * a.fo_items_stride;
-    uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
     const int b0 = tid * kPer;
-    uint32_t c[kPer];
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) c[j] = r.bin[b0 + j];
+    auto at_bin = [](int b) { return b + (b >> 4); };
+    for (int i = tid; i < kBins; i += kFT) sh.c[at_bin(i)] = r.bin[i];
     float vmax;
     uint32_t shift;
     fb_bin_shape(r, parts, kBins, p, vmax, shift);
     const double S = wave::sum_f64(lane < parts ? r.psum[lane] : 0.0);
     if (tid == 0) {
-        s_bad = 0u;
-        s_cut = s_stop = s_first = 0xffffffffu;
-        s_last = 0u;
-        s_cut_lo = s_cut_hi = 0.0;
-        s_stop_q = 0.0f;
-        s_off0 = s_off1 = 0u;
+        sh.bad = 0u;
+        sh.cut = sh.stop = sh.first = 0xffffffffu;
+        sh.last = 0u;
+        sh.cut_lo = sh.cut_hi = 0.0;
+        sh.stop_q = 0.0f;
+        sh.off0 = sh.off1 = 0u;
     }
-    for (int i = tid; i < kBins / 32; i += kFT) smask[i] = 0u;
+    for (int i = tid; i < kBins / 32; i += kFT) sh.mask[i] = 0u;
+    __syncthreads();
+    const float inv = static_cast<float>(1.0 / S);
+    const float minimum = inv * p.min_p;  // generation.cpp:104, probs[0] = 1 * inv
+    const double tp = p.top_p == p.top_p ? static_cast<double>(p.top_p) : 1e30;
+    const float tiny = S >= 0.5 && S < 0x1p60 ? __builtin_ldexpf(1.0f, min(sum_exp(S) - 29, 0)) : 1.0f;
     // The exps of bin b: [lo_bits, hi_bits] (the last bin: from 0).
-    auto hi_pe = [&](int j) { return u2f(kOne - (static_cast<uint32_t>(b0 + j) << shift)); };
-    auto lo_pe = [&](int j) {
-        return b0 + j == kBins - 1 ? 0.0f : u2f(kOne - (static_cast<uint32_t>(b0 + j + 1) << shift) + 1u);
+    auto hi_pe = [&](int b) { return u2f(kOne - (static_cast<uint32_t>(b) << shift)); };
+    auto lo_pe = [&](int b) { return b == kBins - 1 ? 0.0f : u2f(kOne - (static_cast<uint32_t>(b + 1) << shift) + 1u); };
+    auto mid = [&](int b) { return 0.5f * (lo_pe(b) * inv + hi_pe(b) * inv); };
+    auto rounded = [&](int b, float c, double acc) {  // bin b's addends in the binade of acc
+        const int e = max(fb_expo(acc), 64);          // (below 2^-63 nothing rounds)
+        return c * __builtin_ldexpf(__builtin_rintf(__builtin_ldexpf(mid(b), 150 - e)), e - 150);
+    };
+    // f(bin, its padded index, its count) for this thread's bins that hold any.
+    auto each = [&](auto&& f) {
+        constexpr int kBatch = kPer < 4 ? kPer : 4;
+#pragma unroll 1
+        for (int j = 0; j < kPer; j += kBatch) {
+            uint32_t c[kBatch];
+#pragma unroll
+            for (int v = 0; v < kBatch; ++v) c[v] = sh.c[at_bin(b0 + j + v)];
+#pragma unroll
+            for (int v = 0; v < kBatch; ++v)
+                if (c[v] != 0u) f(b0 + j + v, at_bin(b0 + j + v), c[v]);
+        }
     };
     uint32_t fine = 0, n_t = 0;
-    const float tiny = S >= 0.5 && S < 0x1p60 ? __builtin_ldexpf(1.0f, min(sum_exp(S) - 29, 0)) : 1.0f;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        n_t += c[j];
-        if (lo_pe(j) < tiny) fine += c[j];
-    }
+    double t = 0.0;
+    uint32_t low = 0xffffffffu;  // the min-p cut lies in the first bin with a probability below it
+    each([&](int b, int, uint32_t c) {
+        n_t += c;
+        if (lo_pe(b) < tiny) fine += c;
+        if (lo_pe(b) * inv < minimum) low = min(low, static_cast<uint32_t>(b));
+        t += static_cast<double>(static_cast<float>(c) * mid(b));
+    });
+    if (low != 0xffffffffu) atomicMin(&sh.cut, low);
     uint32_t total, n_fine;
-    uint32_t before = fb_scan_u32(n_t, su, total);  // elements before this thread's bins
-    (void)fb_scan_u32(fine, su, n_fine);
+    const uint32_t before = fb_scan_u32<kFW>(n_t, sh.su, total);  // elements before this thread's bins
+    (void)fb_scan_u32<kFW>(fine, sh.su, n_fine);
     const float inv_temp = 1.0f / p.temperature;
     const bool fits = inv_temp > 0.0f && inv_temp < __builtin_inff() && vmax > -__builtin_inff() &&
                       vmax < __builtin_inff() && total == static_cast<uint32_t>(V) && den_rounds_alike(S, n_fine, V);
@@ -408,87 +465,50 @@ __global__ __launch_bounds__(kFT) void fb_plan_kernel(DevArgs a, int parts) {
         if (tid == 0) meta[kMetaStatus] = kStatusToSort;
         return;
     }
-    const float inv = static_cast<float>(1.0 / S);
-    const float minimum = inv * p.min_p;  // generation.cpp:104, probs[0] = 1 * inv
-    const double tp = p.top_p == p.top_p ? static_cast<double>(p.top_p) : 1e30;
-    // The min-p cut lies in the first bin with a probability below it.
-    {
-        uint32_t first = 0xffffffffu;
-#pragma unroll
-        for (int j = kPer - 1; j >= 0; --j)
-            if (c[j] && lo_pe(j) * inv < minimum) first = static_cast<uint32_t>(b0 + j);
-        if (first != 0xffffffffu) atomicMin(&s_cut, first);
-    }
-    // The float sum before each bin: the exact sum first (x0), for the
-    // binades, then with every addend rounded as it is there (a0). The bins'
-    // own terms are formed again in each sweep, from a copy of inv that the
-    // compiler cannot see through: kept, they spill.
-    auto mid = [&](int j, float iv) {
-        return 0.5 * (static_cast<double>(lo_pe(j) * iv) + static_cast<double>(hi_pe(j) * iv));
-    };
-    auto rounded = [&](int j, float iv, double acc) {  // bin j's addends in the binade of acc
-        const int e = max(fb_expo(acc), 1);
-        return c[j] * __builtin_ldexp(__builtin_rint(__builtin_ldexp(mid(j, iv), 150 - e)), e - 150);
-    };
-    auto opaque = [](float v) {
-        asm volatile("" : "+v"(v));
-        return v;
-    };
-    double x0, a0, w0, all;
-    {
-        double t = 0.0;
-        float iv = opaque(inv);
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) t += c[j] * mid(j, iv);
-        x0 = fb_scan_f64(t, sd, all);
-        double x = x0;
-        t = 0.0;
-        iv = opaque(inv);
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            const double m = c[j] * mid(j, iv);
-            t += rounded(j, iv, x + 0.5 * m);
-            x += m;
-        }
-        a0 = fb_scan_f64(t, sd, all);
-    }
-    // f(j, inv, the sum before bin j, the sum after it)
+    // The float sum before each bin: the exact sum first (x), for the binades,
+    // then with every addend rounded as it is there (A). The bins' middles miss
+    // the exact sum mostly where few large addends hold most of it, in the head
+    // (always replayed): the bins after it begin that much later.
+    double all;
+    double x = fb_scan_f64<kFW>(t, sh.sd, all);
+    const double corr = S * static_cast<double>(inv) - all;
+    x += corr;
+    t = 0.0;
+    each([&](int b, int i, uint32_t c) {
+        const double m = static_cast<double>(static_cast<float>(c) * mid(b));
+        const float g = rounded(b, static_cast<float>(c), x + 0.5 * m);
+        sh.w[i] = f2u(g);
+        t += static_cast<double>(g);
+        x += m;
+    });
+    const double a0 = corr + fb_scan_f64<kFW>(t, sh.sd, all);
+    all += corr;
+    // f(bin, index, count, the sum before the bin, the sum after it)
     auto sweep = [&](auto&& f) {
-        double x = x0, A = a0;
-        const float iv = opaque(inv);
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            const double m = c[j] * mid(j, iv);
-            const double A1 = A + rounded(j, iv, x + 0.5 * m);
-            f(j, iv, A, A1);
-            x += m;
+        double A = a0;
+        each([&](int b, int i, uint32_t c) {
+            const double A1 = A + static_cast<double>(u2f(sh.w[i]));
+            f(b, i, c, A, A1);
             A = A1;
-        }
-    };
-    {
-        const uint32_t cut = s_cut;  // (written before the scans' barriers)
-        sweep([&](int j, float, double A, double A1) {
-            const uint32_t b = static_cast<uint32_t>(b0 + j);
-            if (b == cut) {
-                s_cut_lo = A;
-                s_cut_hi = A1;
-            }
-            if (c[j] && A1 * (1.0 + kFbDrift) >= tp && A * (1.0 + kFbDrift) < tp) atomicMin(&s_stop, b);
         });
-        if (cut == 0xffffffffu && tid == 0) s_cut_lo = s_cut_hi = all;
-    }
+    };
+    const uint32_t cut = sh.cut;  // (written before the scans' barriers)
+    sweep([&](int b, int, uint32_t, double A, double A1) {
+        if (static_cast<uint32_t>(b) == cut) {
+            sh.cut_lo = A;
+            sh.cut_hi = A1;
+        }
+        if (A1 * (1.0 + kFbDrift) >= tp && A * (1.0 + kFbDrift) < tp) atomicMin(&sh.stop, static_cast<uint32_t>(b));
+    });
+    if (cut == 0xffffffffu && tid == 0) sh.cut_lo = sh.cut_hi = all;
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kPer; ++j)
-        if (static_cast<uint32_t>(b0 + j) == s_stop) s_stop_q = hi_pe(j) * inv;
-    __syncthreads();
-    const uint32_t cut = s_cut;
     // The mass the draw is taken of: top_p and less than the stopping addend
     // more, or the sum before the cut; at least the first probability.
     const double q_first = static_cast<double>(inv);
-    double mass_lo = tp < s_cut_lo ? tp : s_cut_lo;
-    const double over = tp + static_cast<double>(s_stop_q);
-    double mass_hi = over < s_cut_hi ? over : s_cut_hi;
+    double mass_lo = tp < sh.cut_lo ? tp : sh.cut_lo;
+    const uint32_t stop = sh.stop;
+    const double over = tp + (stop != 0xffffffffu ? static_cast<double>(hi_pe(static_cast<int>(stop)) * inv) : 0.0);
+    double mass_hi = over < sh.cut_hi ? over : sh.cut_hi;
     if (!(mass_lo > q_first)) {
         mass_lo = q_first;
         mass_hi = max(mass_hi, 2.0 * q_first);
@@ -497,116 +517,140 @@ __global__ __launch_bounds__(kFT) void fb_plan_kernel(DevArgs a, int parts) {
     const double c_lo = u * mass_lo * (1.0 - 2.0 * kFbDrift), c_hi = u * mass_hi * (1.0 + 2.0 * kFbDrift);
     const double c_mid = 0.5 * (c_lo + c_hi);
     // What the walk has taken off before each bin.
-    {
-        double t = 0.0;
-        sweep([&](int j, float iv, double A, double A1) { t += rounded(j, iv, c_mid - 0.5 * (A + A1)); });
-        w0 = fb_scan_f64(t, sd, all);
-    }
-    uint32_t n_items = 0, n_seg = 0;
-    uint32_t expand = 0, visit = 0;
-    uint32_t tag[kPer];
+    // (threads whose bins no chain reaches have nothing more to find)
+    const bool live = n_t != 0u && (before < kFbHead || (a0 * (1.0 - kFbDrift) < tp && static_cast<uint32_t>(b0) <= cut));
+    t = 0.0;
+    if (live) sweep([&](int b, int, uint32_t c, double A, double A1) {
+        t += static_cast<double>(rounded(b, static_cast<float>(c), c_mid - 0.5 * (A + A1)));
+    });
+    double W = corr + fb_scan_f64<kFW>(t, sh.sd, all);
+    // What each bin is: seen by the chains, expanded, replayed. A seen bin's
+    // word then holds its record's info when it is expanded, else the ulps it
+    // adds per addend (24 bits) and the walk's exponent.
+    uint32_t n_items = 0, n_seg = 0, n_elem = 0;
+    double s_cum = 0.0, s_walk = 0.0;  // the unexpanded bins' ulps
     uint32_t at = before;
-    double W = w0;
-    sweep([&](int j, float iv, double A, double A1) {
-        const uint32_t b = static_cast<uint32_t>(b0 + j);
-        const double W1 = W + rounded(j, iv, c_mid - 0.5 * (A + A1));
-        tag[j] = 0u;
-        if (c[j] != 0u) {
-            const float qh = hi_pe(j) * iv, ql = lo_pe(j) * iv;
-            const bool head = at < kFbHead;
-            const double a_lo = A * (1.0 - kFbDrift), a_hi = A1 * (1.0 + kFbDrift);
-            const bool seen = head || (a_lo < tp && b <= cut);
-            bool ex = head || b == cut || a_hi >= tp;
+    uint32_t seen = 0;  // how many of this thread's bins with tokens are (a prefix of them)
+    uint32_t expo_end = 0;
+    // The walk's ulps per addend of an unexpanded bin.
+    auto walk_ulps = [&](int b, int ew) -> uint32_t {
+        return ew ? static_cast<uint32_t>(__builtin_floorf(__builtin_ldexpf(hi_pe(b) * inv, 150 - ew) + 0.5f)) : 0u;
+    };
+    if (live) sweep([&](int b, int i, uint32_t c, double A, double A1) {
+        const double W1 = W + static_cast<double>(rounded(b, static_cast<float>(c), c_mid - 0.5 * (A + A1)));
+        const bool head = at < kFbHead;
+        const double a_lo = A * (1.0 - kFbDrift), a_hi = A1 * (1.0 + kFbDrift);
+        if (head || (a_lo < tp && static_cast<uint32_t>(b) <= cut)) {
+            const float qh = hi_pe(b) * inv, ql = lo_pe(b) * inv;
+            const bool edge = head || static_cast<uint32_t>(b) == cut || a_hi >= tp;
             const int ea = fb_expo(a_lo);
-            ex = ex || ea != fb_expo(a_hi) || ea == 0 || !fb_alike(ql, qh, ea);
-            tag[j] = static_cast<uint32_t>(ea);
+            uint32_t dc = 0, dw = 0;
+            const bool rc = edge || ea != fb_expo(a_hi) || ea == 0;
+            bool ex = rc || !fb_alike(ql, qh, ea, dc);
+            int ew = 0;
+            bool rw = false;
             const double w_hi = c_hi * (1.0 + kFbDrift) - W, w_lo = c_lo - c_hi * kFbDrift - W1;
             if (w_hi > 0.0) {
-                const int ew = fb_expo(w_hi);
-                if (!(w_lo > 0.0)) {
-                    ex = true;
-                    if (seen) {  // the walk may stop here
-                        atomicMin(&s_first, b);
-                        atomicMax(&s_last, b);
-                    }
-                } else {
-                    ex = ex || ew != fb_expo(w_lo) || !fb_alike(ql, qh, ew);
+                ew = fb_expo(w_hi);
+                const bool draw = !(w_lo > 0.0);  // the walk may stop here
+                rw = edge || draw || ew != fb_expo(w_lo);
+                ex = ex || rw || !fb_alike(ql, qh, ew, dw);
+                if (draw) {
+                    atomicMin(&sh.first, static_cast<uint32_t>(b));
+                    atomicMax(&sh.last, static_cast<uint32_t>(b));
                 }
-                tag[j] |= static_cast<uint32_t>(ew) << 8;
             }
-            if (seen) {
-                visit |= 1u << j;
-                if (ex) {
-                    expand |= 1u << j;
-                    n_items += c[j];
-                    ++n_seg;
-                    if (c[j] > kFbSegMost) s_bad = 1u;
-                } else {
-                    ++n_items;
-                }
+            ++seen;
+            n_elem += c;
+            expo_end = static_cast<uint32_t>(fb_expo(A1 * (1.0 - kFbDrift)));
+            if (ex) {
+                n_items += c;
+                ++n_seg;
+                if (c > kFbSegMost && (rc || rw)) sh.bad = 1u;
+                atomicOr(&sh.mask[b >> 5], 1u << (b & 31));
+                sh.w[i] = static_cast<uint32_t>(ea) | (static_cast<uint32_t>(ew) << 8) | (rc ? kSegReplayCum : 0u) |
+                          (rw ? kSegReplayWalk : 0u) | (ew ? kSegInWalk : 0u);
+            } else {
+                s_cum += static_cast<double>(c) * static_cast<double>(dc);
+                s_walk += static_cast<double>(c) * static_cast<double>(dw);
+                sh.w[i] = dc | (static_cast<uint32_t>(ew) << 24);
             }
         }
-        at += c[j];
+        at += c;
         W = W1;
     });
-    uint32_t G, segs;
-    uint32_t off = fb_scan_u32(n_items, su, G);
-    uint32_t seg = fb_scan_u32(n_seg, su, segs);
-    if (s_bad || static_cast<int64_t>(G) + 1 > fb_half(a) || segs > static_cast<uint32_t>(kFbSegs)) {
+    uint32_t G, segs, elems;
+    uint32_t off = fb_scan_u32<kFW>(n_items, sh.su, G);
+    uint32_t seg = fb_scan_u32<kFW>(n_seg, sh.su, segs);
+    (void)fb_scan_u32<kFW>(n_elem, sh.su, elems);
+    double cum_all, walk_all;
+    double cum = fb_scan_f64<kFW>(s_cum, sh.sd, cum_all);
+    double walk = fb_scan_f64<kFW>(s_walk, sh.sd, walk_all);
+    if (sh.bad || static_cast<int64_t>(G) + 1 > fb_half(a) || segs > static_cast<uint32_t>(kFbSegs)) {
         if (tid == 0) meta[kMetaStatus] = kStatusToSort;
         return;
     }
+    const uint32_t draw0 = sh.first, draw1 = sh.last;
     at = before;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const uint32_t b = static_cast<uint32_t>(b0 + j);
-        if ((visit >> j) & 1u) {
-            if (b == s_first) s_off0 = off;
-            if ((expand >> j) & 1u) {
+    if (seen != 0u) {
+        uint32_t left = seen;
+        each([&](int b, int i, uint32_t c) {
+            if (left == 0u) return;
+            --left;
+            const uint32_t w = sh.w[i];
+            if (static_cast<uint32_t>(b) == draw0) sh.off0 = off;
+            if ((sh.mask[b >> 5] >> (b & 31)) & 1u) {
                 r.bin[b] = off;
-                r.seg[3 * seg] = off;
-                r.seg[3 * seg + 1] = c[j];
-                r.seg[3 * seg + 2] = at;
+                r.seg[seg] = FbSeg{off, c, at, w, cum, walk, 0u, 0u};
                 ++seg;
-                off += c[j];
-                atomicOr(&smask[b >> 5], 1u << (b & 31u));
+                off += c;
             } else {
-                items[off] = kFbRegular | tag[j];
-                aux[off] = hi_pe(j);
-                pre[off] = at;
-                ++off;
+                cum += static_cast<double>(c) * static_cast<double>(w & 0xffffffu);
+                walk += static_cast<double>(c) * static_cast<double>(walk_ulps(b, static_cast<int>(w >> 24)));
             }
-            if (b == s_last) s_off1 = off;
-            if (off == G) pre[G] = at + c[j];
-        }
-        at += c[j];
+            if (static_cast<uint32_t>(b) == draw1) sh.off1 = off;
+            at += c;
+        });
+        if (at == elems) r.seg[segs] = FbSeg{G, 0u, elems, expo_end | kSegReplayCum, cum_all, walk_all, 0u, 0u};  // the list's end
     }
     __syncthreads();
-    for (int i = tid; i < kBins / 32; i += kFT) r.mask[i] = smask[i];
+    for (int i = tid; i < kBins / 32; i += kFT) r.mask[i] = sh.mask[i];
     if (tid == 0) {
+        const bool none = draw0 == 0xffffffffu;
         r.scal[kScShift] = shift;
         r.scal[kScInv] = f2u(inv);
-        r.scal[kScDrawBin] = s_first == 0xffffffffu ? 0u : s_first;
-        r.scal[kScDrawItem] = s_off0;
-        r.scal[kScDrawEnd] = s_first == 0xffffffffu ? 0u : s_off1;
+        r.scal[kScDrawBin] = none ? 0u : draw0;
+        r.scal[kScDrawItem] = sh.off0;
+        r.scal[kScDrawEnd] = none ? 0u : sh.off1;
         r.scal[kScSegs] = segs;
+        // whether the list ends where the reference's sums do: the row's end,
+        // or the bin of the min-p cut
+        r.scal[kScCut] = elems == static_cast<uint32_t>(V) || (cut != 0xffffffffu && sh.cut_lo * (1.0 - kFbDrift) < tp) ? 1u : 0u;
         meta[kMetaItems] = G;
         meta[kMetaStatus] = kStatusOk;
     }
 }
 
 // 4. The expanded bins' tokens to their items, in no order, and the sum of the
-//    probabilities of the bins before the draw's. A streaming read of the
-//    exps; about one token in ten is expanded in near-uniform rows.
-__global__ __launch_bounds__(kFT) void fb_collect_kernel(DevArgs a) {
-    __shared__ uint32_t smask[kFbMaxBins / 32];
-    __shared__ double sums[kFW];
-    const int row = blockIdx.y, part = blockIdx.x, parts = gridDim.x, tid = threadIdx.x;
+//    probabilities of the bins before the draw's. Streaming reads of the exps;
+//    about one token in ten is expanded in near-uniform rows. Places are taken
+//    from LDS counters: a part counts its tokens of each expanded bin first and
+//    takes its share of the bin's items with one global atomic (the part is in
+//    cache for its second read). With an atomic per token, 256 flat rows took
+//    204 us and 64 peaked rows 27.
+struct CollectShared {
+    uint32_t next[kFbMaxBins];
+    uint32_t mask[kFbMaxBins / 32];
+    double sums[kFW];
+};
+__device__ __forceinline__ void fb_collect(const DevArgs& a, int row, int part, int parts, CollectShared& sh) {
+    const int tid = threadIdx.x;
     ge_sample_params p;
     if (!fb_serves(a, row, p) || fb_meta(a, row)[kMetaStatus] != kStatusOk) return;
     const int bins = fb_bins(a.vocab);
     const FbRow r = fb_row(a, row, bins);
-    for (int i = tid; i < bins / 32; i += kFT) smask[i] = r.mask[i];
+    for (int i = tid; i < bins / 32; i += kFT) sh.mask[i] = r.mask[i];
+    for (int i = tid; i < bins; i += kFT) sh.next[i] = parts == 1 ? r.bin[i] : 0u;
     const uint32_t shift = r.scal[kScShift];
     const float inv = u2f(r.scal[kScInv]);
     const uint32_t draw = r.scal[kScDrawBin];
@@ -615,6 +659,23 @@ __global__ __launch_bounds__(kFT) void fb_collect_kernel(DevArgs a) {
     fb_part(a, part, parts, lo, hi);
     const float* pes = fb_exp_array(a, row);
     uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
+    auto expanded = [&](uint32_t b) { return ((sh.mask[b >> 5] >> (b & 31u)) & 1u) != 0u; };
+    if (parts > 1) {
+        fb_stream<4>(pes, true, lo, hi, tid, [&](int, float x0, float x1, float x2, float x3, int n) {
+            const float x[4] = {x0, x1, x2, x3};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t b = fb_bin(x[j], shift, static_cast<uint32_t>(bins));
+                if (j < n && expanded(b)) atomicAdd(&sh.next[b], 1u);
+            }
+        });
+        __syncthreads();
+        for (int i = tid; i < bins; i += kFT) {
+            const uint32_t c = sh.next[i];
+            if (c) sh.next[i] = atomicAdd(&r.bin[i], c);
+        }
+        __syncthreads();
+    }
     double sum = 0.0;
     fb_stream<4>(pes, true, lo, hi, tid, [&](int i, float x0, float x1, float x2, float x3, int n) {
         const float x[4] = {x0, x1, x2, x3};
@@ -623,56 +684,109 @@ __global__ __launch_bounds__(kFT) void fb_collect_kernel(DevArgs a) {
             if (j < n) {
                 const uint32_t b = fb_bin(x[j], shift, static_cast<uint32_t>(bins));
                 if (b < draw) sum += static_cast<double>(x[j] * inv);
-                if ((smask[b >> 5] >> (b & 31u)) & 1u) {
-                    const uint32_t at = atomicAdd(&r.bin[b], 1u);
+                if (expanded(b)) {
+                    const uint32_t at = atomicAdd(&sh.next[b], 1u);
                     items[at] = (static_cast<uint64_t>(f2u(x[j])) << 32) | (0xffffffffu - static_cast<uint32_t>(i + j));
                 }
             }
         }
     });
     sum = wave::sum_f64(sum);
-    if ((tid & 63) == 0) sums[tid >> 6] = sum;
+    if ((tid & 63) == 0) sh.sums[tid >> 6] = sum;
     __syncthreads();
     if (tid == 0) {
         double t = 0.0;
-        for (int w = 0; w < kFW; ++w) t += sums[w];
+        for (int w = 0; w < kFW; ++w) t += sh.sums[w];
         r.pbef[part] = t;
     }
 }
 
-// 5. The tokens of each expanded bin by (exp descending, index ascending), with
-//    the items' first elements: one wave per bin by counting the larger keys
-//    (every lane's up to eight keys against an LDS broadcast), the workgroup
-//    by a bitonic sort for the rare larger ones.
-constexpr int kOT = 256;
-constexpr int kOW = kOT / 64;
-__global__ __launch_bounds__(kOT) void fb_order_kernel(DevArgs a) {
-    __shared__ uint64_t stage[kFbSegMost];
-    static_assert(kOW * kFbWaveSeg <= static_cast<int>(kFbSegMost), "the waves' shares");
-    const int row = blockIdx.y, tid = threadIdx.x, lane = __lane_id(), wave = tid >> 6;
+// 5. Each expanded bin: the ulps its tokens add where it is not replayed (a
+//    bin with a tie among them is replayed after all), and a replayed bin's
+//    tokens by (exp descending, index ascending): one wave per bin by counting
+//    the larger keys (every lane's up to eight keys against an LDS broadcast),
+//    the workgroup by a bitonic sort for the rare larger ones.
+struct OrderShared {
+    uint64_t stage[kFbSegMost];
+};
+template <int kThreads>
+__device__ __forceinline__ void fb_order(const DevArgs& a, int row, int block, int blocks, OrderShared& sh) {
+    constexpr int kWaves = kThreads / 64;
+    constexpr int kMy = std::min(kFbWaveSeg, static_cast<int>(kFbSegMost) / kWaves) / 64;  // keys per lane
+    constexpr uint32_t kWaveSeg = kMy * 64;
+    const int tid = threadIdx.x, lane = __lane_id(), wave = tid >> 6;
     ge_sample_params p;
-    if (!fb_serves(a, row, p) || fb_meta(a, row)[kMetaStatus] != kStatusOk) return;
+    uint32_t* meta = fb_meta(a, row);
+    if (!fb_serves(a, row, p) || meta[kMetaStatus] != kStatusOk) return;
     const FbRow r = fb_row(a, row, fb_bins(a.vocab));
     const int segs = static_cast<int>(r.scal[kScSegs]);
+    const float inv = u2f(r.scal[kScInv]);
     uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
-    float* aux = a.fo_aux + static_cast<int64_t>(row) * a.fo_items_stride;
-    uint32_t* pre = a.fo_pre + static_cast<int64_t>(row) * a.fo_items_stride;
-    auto place = [&](uint32_t item, uint32_t elem, uint64_t key) {
-        items[item] = key;
-        aux[item] = u2f(static_cast<uint32_t>(key >> 32));
-        pre[item] = elem;
-    };
-    uint64_t* mine = stage + wave * kFbWaveSeg;
+    uint64_t* mine = sh.stage + wave * kWaveSeg;
     bool large = false;
-    for (int s = blockIdx.x * kOW + wave; s < segs; s += gridDim.x * kOW) {
-        const uint32_t off = r.seg[3 * s], n = r.seg[3 * s + 1], first = r.seg[3 * s + 2];
+    // A wave reads 64 records at once (lane l: its l-th, the waves taking bins
+    // in turn) and passes those with nothing to do, the single tokens of the
+    // head above all; the next bin's first keys are in flight while one is
+    // worked on.
+    auto work = [&](uint32_t info, uint32_t n) {
+        return n > 1u || !(info & kSegReplayCum) || ((info & kSegInWalk) && !(info & kSegReplayWalk));
+    };
+    const int turn = blocks * kWaves;
+    for (int c0 = block * kWaves + wave; c0 < segs; c0 += turn * 64) {
+      const int mine_s = c0 + lane * turn;
+      const bool have = mine_s < segs;
+      const uint32_t r_off = have ? r.seg[mine_s].item : 0u, r_n = have ? r.seg[mine_s].n : 0u;
+      const uint32_t r_info = have ? r.seg[mine_s].info : 0u;
+      uint64_t todo = __ballot(have && work(r_info, r_n));
+      auto first_keys = [&](int l) {
+          const uint32_t o = wave::readlane(r_off, l), m = wave::readlane(r_n, l);
+          return items[o + min(static_cast<uint32_t>(lane), m - 1u)];
+      };
+      uint64_t next = todo ? first_keys(__builtin_ctzll(todo)) : 0ull;
+      while (todo) {
+        const int l = static_cast<int>(__builtin_ctzll(todo));
+        todo &= todo - 1ull;
+        const int s = c0 + l * turn;
+        const uint32_t off = wave::readlane(r_off, l), n = wave::readlane(r_n, l);
+        uint32_t info = wave::readlane(r_info, l);
+        const bool sum_c = !(info & kSegReplayCum);
+        const bool sum_w = (info & kSegInWalk) && !(info & kSegReplayWalk);
+        const uint64_t key0 = static_cast<uint32_t>(lane) < n ? next : 0ull;
+        if (todo) next = first_keys(__builtin_ctzll(todo));
+        if (sum_c || sum_w) {
+            const int uc = static_cast<int>(info & 0xffu) - 150, uw = static_cast<int>((info >> 8) & 0xffu) - 150;
+            uint32_t tc = 0, tw = 0;
+            bool oc = false, ow = false;  // a tie, an addend past the binade, or a sum past it
+            for (uint32_t i = static_cast<uint32_t>(lane); i < n; i += 64u) {
+                const uint64_t key = i < 64u ? key0 : items[off + i];
+                const uint32_t qb = f2u(u2f(static_cast<uint32_t>(key >> 32)) * inv);
+                uint32_t D;
+                bool tie, big;
+                chain::step_bits(qb, uc, D, tie, big);
+                tc += min(D, 0x1000000u);
+                oc = oc || tie || big || tc > 0x1000000u;
+                tc = min(tc, 0x1000000u);
+                chain::step_bits(qb, uw, D, tie, big);
+                tw += min(D, 0x1000000u);
+                ow = ow || tie || big || tw > 0x1000000u;
+                tw = min(tw, 0x1000000u);
+            }
+            // (a lane's sum stays below 2^25, so the wave's fits 31 bits)
+            if (sum_c && __ballot(oc)) info |= kSegReplayCum;
+            if (sum_w && __ballot(ow)) info |= kSegReplayWalk;
+            const uint32_t dc = wave::incl_add(tc), dw = wave::incl_add(tw);
+            if (lane == 63) {
+                r.seg[s].info = info;
+                r.seg[s].scum = dc;
+                r.seg[s].swalk = dw;
+            }
+        }
+        if (!(info & (kSegReplayCum | kSegReplayWalk))) continue;
         if (n <= 64u) {
-            const uint64_t key = static_cast<uint32_t>(lane) < n ? items[off + lane] : 0ull;
             uint32_t rank = 0;
-            for (uint32_t j = 0; j < n; ++j) rank += wave::readlane64(key, static_cast<int>(j)) > key ? 1u : 0u;
-            if (static_cast<uint32_t>(lane) < n) place(off + rank, first + rank, key);
-        } else if (n <= static_cast<uint32_t>(kFbWaveSeg)) {
-            constexpr int kMy = kFbWaveSeg / 64;
+            for (uint32_t j = 0; j < n; ++j) rank += wave::readlane64(key0, static_cast<int>(j)) > key0 ? 1u : 0u;
+            if (static_cast<uint32_t>(lane) < n) items[off + rank] = key0;
+        } else if (n <= kWaveSeg) {
             uint64_t key[kMy];
             uint32_t rank[kMy];
 #pragma unroll
@@ -691,190 +805,356 @@ __global__ __launch_bounds__(kOT) void fb_order_kernel(DevArgs a) {
             }
 #pragma unroll
             for (int v = 0; v < kMy; ++v)
-                if (static_cast<uint32_t>(v) * 64u + static_cast<uint32_t>(lane) < n) place(off + rank[v], first + rank[v], key[v]);
+                if (static_cast<uint32_t>(v) * 64u + static_cast<uint32_t>(lane) < n) items[off + rank[v]] = key[v];
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         } else {
             large = true;
+            if (n > kFbSegMost && lane == 0) meta[kMetaStatus] = kStatusToSort;
         }
+      }
     }
+    __builtin_amdgcn_s_waitcnt(0);  // the flags written above are read below by every wave
     if (__syncthreads_or(large ? 1 : 0) == 0) return;
-    for (int s0 = blockIdx.x * kOW; s0 < segs; s0 += gridDim.x * kOW) {
-        for (int s = s0; s < min(s0 + kOW, segs); ++s) {
-            const uint32_t off = r.seg[3 * s], n = r.seg[3 * s + 1], first = r.seg[3 * s + 2];
-            if (n <= static_cast<uint32_t>(kFbWaveSeg)) continue;  // (block-uniform)
+    for (int s0 = block * kWaves; s0 < segs; s0 += turn) {
+        for (int s = s0; s < min(s0 + kWaves, segs); ++s) {
+            const uint32_t off = r.seg[s].item, n = r.seg[s].n;
+            // (block-uniform; the flags as this workgroup's waves left them)
+            const uint32_t info = ld_l2(&r.seg[s].info);
+            if (n <= kWaveSeg || n > kFbSegMost || !(info & (kSegReplayCum | kSegReplayWalk))) continue;
             uint32_t n2 = 1;
             while (n2 < n) n2 <<= 1;
             __syncthreads();
-            for (uint32_t i = tid; i < n2; i += kOT) stage[i] = i < n ? items[off + i] : 0ull;
+            for (uint32_t i = tid; i < n2; i += kThreads) sh.stage[i] = i < n ? items[off + i] : 0ull;
             for (uint32_t size = 2; size <= n2; size <<= 1) {
                 for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
                     __syncthreads();
-                    for (uint32_t q = tid; q < n2 / 2; q += kOT) {
+                    for (uint32_t q = tid; q < n2 / 2; q += kThreads) {
                         const uint32_t i = 2u * q - (q & (stride - 1u));
-                        const uint64_t x = stage[i], y = stage[i + stride];
+                        const uint64_t x = sh.stage[i], y = sh.stage[i + stride];
                         const bool desc = (i & size) == 0u;
                         if (desc ? x < y : x > y) {
-                            stage[i] = y;
-                            stage[i + stride] = x;
+                            sh.stage[i] = y;
+                            sh.stage[i + stride] = x;
                         }
                     }
                 }
             }
             __syncthreads();
-            for (uint32_t i = tid; i < n; i += kOT) place(off + i, first + i, stage[i]);
+            for (uint32_t i = tid; i < n; i += kThreads) items[off + i] = sh.stage[i];
         }
     }
 }
 
-// 6. The chains (generation.cpp:103-126) over the items with the whole
-//    workgroup, the checks of the plan, and the token. Latency-bound: a pass
-//    of block_chain per binade change, most of them 64-item probes at the head.
-constexpr int kDrawThreads = 512;
-constexpr int kDrawWaves = kDrawThreads / 64;
-constexpr int kDrawLog = 96;   // binade changes logged per chain
-constexpr int kDrawTies = 4096;  // tokens of one exp (kFbSegMost)
+// 6. The chains (generation.cpp:103-126): the replayed bins' probabilities in
+//    LDS lists, one for the cumulative and one for the walk, cut into regions
+//    of consecutive elements; the ulps of the bins between two regions are
+//    added at once. One wave takes the lists 64 elements a step. Then the
+//    near-boundary flag and the token. Latency-bound: about 150 steps of
+//    dependent work per chain for near-uniform rows.
+constexpr int kDrawList = 8192;     // replayed elements of one chain
+constexpr int kDrawRegions = 512;   // their regions
+constexpr int kDrawTies = 4096;     // tokens of one exp (kFbSegMost)
 
+struct DrawList {
+    union {
+        uint32_t q[kDrawList];      // the probabilities' bits
+        uint64_t tie[kDrawTies];    // (once the chains are done)
+    };
+    double before[kDrawRegions + 1];   // ulps of the bins before the region, from the row's start
+    uint32_t pos[kDrawRegions + 1];    // its first list position; [n]: the list's length
+    uint32_t item[kDrawRegions + 1];
+    uint32_t elem[kDrawRegions + 1];
+    uint32_t expo[kDrawRegions + 1];   // the accumulator's binade before it
+    int n;                             // regions
+};
+static_assert(kDrawList * 4 == kDrawTies * 8, "the union");
 struct DrawShared {
-    bchain::Shared<kDrawWaves> bc;
-    uint64_t tie[kDrawTies];
-    int log_item[kDrawLog];
-    uint32_t log_expo[kDrawLog];
-    int log_n;
-    uint32_t bad;
-    double sums[kDrawWaves];
+    DrawList list[2];  // cumulative, walk
+    double sd[16];
+    uint32_t su[16], sr[16];
+    double s;
+    uint32_t keep, pos, item, near_u, ok;
     int32_t token;
 };
 
-// Logs the binade that the accumulator is in after each event item.
-struct DrawLog {
-    DrawShared* sh;
-    int n = 0;
-    __device__ void operator()(int item, double s) {
-        if (threadIdx.x == 0 && n < kDrawLog) {
-            sh->log_item[n] = item;
-            sh->log_expo[n] = static_cast<uint32_t>(fb_expo(s));
+// Both chains' lists from the row's expanded bins: thread t takes consecutive
+// records, and one workgroup scan places its regions and elements. False
+// (block-uniform) when they do not fit.
+template <int kThreads>
+__device__ __forceinline__ bool draw_lists(const FbRow& r, int segs, const uint64_t* items, float inv, DrawShared& sh) {
+    constexpr int kWaves = kThreads / 64;
+    constexpr int kBatch = 4;  // records in flight
+    constexpr uint32_t kReplay[2] = {kSegReplayCum, kSegReplayWalk};
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const int count = segs + 1;  // with the list's end
+    const int per = (count + kThreads - 1) / kThreads;
+    const int s0 = min(tid * per, count), s1 = min(s0 + per, count);
+    // f(record, chain, replayed, begins a region)
+    auto each = [&](auto&& f) {
+        const FbSeg p = r.seg[max(s0 - 1, 0)];
+        bool prev[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) prev[x] = s0 > 0 && (p.info & kReplay[x]) != 0u;
+        uint32_t next = p.elem + p.n;
+        for (int b = s0; b < s1; b += kBatch) {
+            FbSeg g[kBatch];
+#pragma unroll
+            for (int v = 0; v < kBatch; ++v) g[v] = r.seg[min(b + v, count - 1)];  // clamped: no conditional load
+#pragma unroll
+            for (int v = 0; v < kBatch; ++v) {
+                if (b + v >= s1) continue;
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    const bool rep = (g[v].info & kReplay[x]) != 0u;
+                    f(g[v], x, rep, rep && !(prev[x] && next == g[v].elem && g[v].n != 0u));
+                    prev[x] = rep;
+                }
+                next = g[v].elem + g[v].n;
+            }
         }
-        ++n;
+    };
+    double t[2] = {0.0, 0.0};  // the ulps of the expanded bins that are not replayed
+    uint32_t n[2] = {0, 0}, at[2] = {0, 0};
+    each([&](const FbSeg& g, int x, bool rep, bool start) {
+        if (rep) n[x] += g.n;
+        else t[x] += static_cast<double>(x ? g.swalk : g.scum);
+        at[x] += start ? 1u : 0u;
+    });
+    uint32_t n_all[2], r_all[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        const double ti = wave::incl_f64(t[x]);
+        const uint32_t ni = wave::incl_add(n[x]), ri = wave::incl_add(at[x]);
+        if ((tid & 63) == 63) {
+            sh.sd[8 * x + wave] = ti;
+            sh.su[8 * x + wave] = ni;
+            sh.sr[8 * x + wave] = ri;
+        }
+        t[x] = ti - t[x];
+        n[x] = ni - n[x];
+        at[x] = ri - at[x];
     }
-};
+    static_assert(kWaves <= 8, "the scan's words");
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        n_all[x] = r_all[x] = 0;
+        for (int w = 0; w < kWaves; ++w) {
+            if (w < wave) {
+                t[x] += sh.sd[8 * x + w];
+                n[x] += sh.su[8 * x + w];
+                at[x] += sh.sr[8 * x + w];
+            }
+            n_all[x] += sh.su[8 * x + w];
+            r_all[x] += sh.sr[8 * x + w];
+        }
+    }
+    if (max(n_all[0], n_all[1]) > static_cast<uint32_t>(kDrawList) || max(r_all[0], r_all[1]) > static_cast<uint32_t>(kDrawRegions))
+        return false;
+    each([&](const FbSeg& g, int x, bool rep, bool start) {
+        DrawList& l = sh.list[x];
+        if (start) {
+            l.before[at[x]] = t[x] + (x ? g.walk : g.cum);
+            l.pos[at[x]] = n[x];
+            l.item[at[x]] = g.item;
+            l.elem[at[x]] = g.elem;
+            l.expo[at[x]] = x ? (g.info >> 8) & 0xffu : g.info & 0xffu;
+            ++at[x];
+        }
+        if (rep) n[x] += g.n;
+        else t[x] += static_cast<double>(x ? g.swalk : g.scum);
+    });
+    if (tid < 2) {
+        sh.list[tid].n = static_cast<int>(r_all[tid]);
+        sh.list[tid].pos[r_all[tid]] = n_all[tid];
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < n_all[0] + n_all[1]; i += kThreads) {
+        const int x = i < n_all[0] ? 0 : 1;
+        const uint32_t k = x ? i - n_all[0] : i;
+        DrawList& l = sh.list[x];
+        uint32_t lo = 0, hi = r_all[x];  // the region: pos[lo] <= k < pos[lo + 1]
+        while (hi - lo > 1u) {
+            const uint32_t m = (lo + hi) >> 1;
+            if (l.pos[m] <= k) lo = m;
+            else hi = m;
+        }
+        l.q[k] = f2u(u2f(static_cast<uint32_t>(items[l.item[lo] + (k - l.pos[lo])] >> 32)) * inv);
+    }
+    __syncthreads();
+    return true;
+}
 
-__global__ __launch_bounds__(kDrawThreads) void fb_draw_kernel(DevArgs a, int parts) {
-    __shared__ DrawShared sh;
-    const int row = blockIdx.x, tid = threadIdx.x, lane = __lane_id(), wave = tid >> 6;
-    const ge_sample_params pp = a.row_params ? a.row_params[row] : a.params;
+// One wave takes list elements [k, limit) from the accumulator s (asc: s +=
+// q, until s >= thr; desc: s -= q, until s <= q). Returns 1 at a stop (k: its
+// position), 0 at the limit, -1 where the bins between two regions do not fit
+// the binade the plan took them in.
+template <bool kDesc>
+__device__ __forceinline__ int draw_chain(const DrawList& l, uint32_t& k, uint32_t limit, int& region, float& s, float thr) {
+    const int lane = __lane_id();
+    const uint32_t n_all = l.pos[l.n];
+    uint32_t rend = l.pos[region + 1];
+    // (the cumulative ends where a region begins: the bins before it count too)
+    while (k < limit || (!kDesc && k == rend && region + 1 < l.n)) {
+        const chain::StepBits b = chain::binade_bits(f2u(s));
+        const uint32_t tm = kDesc ? 0u : chain::threshold_bits(f2u(thr), b.uexp);
+        if (k == rend) {  // the bins between this region and the next
+            if (region + 1 >= l.n) return -1;
+            const double jump = l.before[region + 1] - l.before[region];
+            if (jump != 0.0) {
+                const double m = static_cast<double>(b.m);
+                if (l.expo[region + 1] != static_cast<uint32_t>(b.uexp + 150)) return -1;
+                if (kDesc ? m - jump < static_cast<double>(b.lo)
+                          : (m + jump > static_cast<double>(chain::kHiF) || m + jump >= static_cast<double>(tm)))
+                    return -1;
+                s = u2f(chain::rebuild_bits(f2u(s), static_cast<uint32_t>(kDesc ? m - jump : m + jump)));
+            }
+            ++region;
+            rend = l.pos[region + 1];
+            continue;
+        }
+        const uint32_t end = min(rend, limit);
+        const bool on = k + static_cast<uint32_t>(lane) < end;
+        const uint32_t qb = l.q[min(k + static_cast<uint32_t>(lane), n_all - 1u)];
+        uint32_t D;
+        bool tie, big;
+        chain::step_bits(qb, b.uexp, D, tie, big);
+        D = on ? D : 0u;
+        const uint32_t incl = wave::incl_add(D);  // at most 64 * 2^24
+        const bool out = kDesc ? b.m < b.lo + incl : (b.m + incl > chain::kHiF || b.m + incl >= tm);
+        const uint64_t ev = __ballot(on && (out || tie || big));
+        if (ev == 0ull) {
+            const uint32_t t = wave::readlane(incl, 63);
+            s = u2f(chain::rebuild_bits(f2u(s), kDesc ? b.m - t : b.m + t));
+            k = min(k + 64u, end);
+            continue;
+        }
+        const int f = static_cast<int>(__builtin_ctzll(ev));
+        const uint32_t t = wave::readlane(incl, f) - wave::readlane(D, f);
+        const float q = u2f(wave::readlane(qb, f));
+        s = u2f(chain::rebuild_bits(f2u(s), kDesc ? b.m - t : b.m + t));
+        k += static_cast<uint32_t>(f);
+        if (kDesc) {
+            if (s <= q) return 1;
+            s = s - q;
+        } else {
+            s = s + q;
+            if (s >= thr) return 1;
+        }
+        ++k;
+    }
+    return 0;
+}
+
+template <int kThreads>
+__device__ __forceinline__ void fb_draw(const DevArgs& a, int row, int parts, DrawShared& sh) {
+    constexpr int kWaves = kThreads / 64;
+    const int tid = threadIdx.x, lane = __lane_id(), wave = tid >> 6;
+    const ge_sample_params p = a.row_params ? a.row_params[row] : a.params;
     uint32_t k;
-    if (!full_order_row(pp, a.vocab, k)) return;
+    if (!full_order_row(p, a.vocab, k)) return;
     if (row_done(a, row)) {
         if (tid == 0) skipped_row(a, row);
         return;
     }
     uint32_t* meta = fb_meta(a, row);
     if (meta[kMetaStatus] != kStatusOk) return;  // the sort-based pass serves the row
-    const ge_sample_params p = pp;
     const int V = a.vocab;
     const FbRow r = fb_row(a, row, fb_bins(V));
-    const int G = static_cast<int>(meta[kMetaItems]);
+    const int segs = static_cast<int>(r.scal[kScSegs]);
     const uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
-    const float* aux = a.fo_aux + static_cast<int64_t>(row) * a.fo_items_stride;
-    const uint32_t* pre = a.fo_pre + static_cast<int64_t>(row) * a.fo_items_stride;
     const float inv = u2f(r.scal[kScInv]);
     const int draw0 = static_cast<int>(r.scal[kScDrawItem]), draw1 = static_cast<int>(r.scal[kScDrawEnd]);
-    if (tid == 0) {
-        sh.bad = 0u;
-        sh.token = -1;
-    }
-    const float q0 = aux[0] * inv;
-    const float minimum = q0 * p.min_p;
-    const uint32_t end = pre[G];
-    // generation.cpp:106-108: the first element e >= 1 with p_e < minimum.
-    uint32_t keff = static_cast<uint32_t>(V);
-    if (q0 < minimum) {
-        keff = 1u;
-    } else if (minimum > 0.0f && G > 1) {
-        const uint32_t pq = wave_partition_point(1u, static_cast<uint32_t>(G), [&](uint32_t i) { return !(aux[i] * inv < minimum); });
-        if (pq < static_cast<uint32_t>(G)) keff = pre[pq];
+    const bool whole = r.scal[kScCut] != 0u;
+    bool ok = draw_lists<kThreads>(r, segs, items, inv, sh);
+    const float u = a.uniforms[row];
+    float choice = 0.0f;
+    if (ok && wave == 0) {
+        const DrawList& lc = sh.list[0];
+        const DrawList& lw = sh.list[1];
+        const uint32_t n_all = lc.pos[lc.n];
+        const float q0 = u2f(lc.q[0]);
+        const float minimum = q0 * p.min_p;
+        bool good = lc.n > 0 && lc.elem[0] == 0u && n_all > 0u;
+        // generation.cpp:106-108: the first element e >= 1 with p_e < minimum
+        // (the list holds the whole bin that has it).
+        uint32_t limit = n_all;
+        if (q0 < minimum) limit = 1u;
+        else if (minimum > 0.0f) limit = wave_partition_point(1u, n_all, [&](uint32_t i) { return !(u2f(lc.q[i]) < minimum); });
+        uint32_t kc = 1u;
+        int rc = 0;
+        float s = q0;
+        uint32_t keep = 1u;
+        if (good && limit > 1u) {
+            const int hit = draw_chain<false>(lc, kc, limit, rc, s, p.top_p);
+            if (hit < 0) good = false;
+            else if (hit == 1) keep = lc.elem[rc] + (kc - lc.pos[rc]) + 1u;
+            else if (limit < n_all || whole) keep = lc.elem[rc] + (kc - lc.pos[rc]);
+            else good = false;  // the list ends before the sums do
+        }
+        // random.h:1864-1871 and generation.cpp:118-124.
+        choice = u * (s - 0.0f) + 0.0f;
+        uint32_t pos = 0u, item = lc.item[0];
+        if (good && choice > 0.0f && choice < __builtin_inff()) {
+            good = lw.n > 0 && lw.elem[0] == 0u;
+            if (good) {
+                // the list's elements before `keep`
+                const uint32_t lr = wave_partition_point(0u, static_cast<uint32_t>(lw.n), [&](uint32_t i) { return lw.elem[i] < keep; }) - 1u;
+                const uint32_t wlim = lw.pos[lr] + min(lw.pos[lr + 1u] - lw.pos[lr], keep - lw.elem[lr]);
+                uint32_t kw = 0u;
+                int rw = 0;
+                float c = choice;
+                const int hit = draw_chain<true>(lw, kw, wlim, rw, c, 0.0f);
+                if (hit == 0) {  // the walk passes every kept element: the last one
+                    good = kw > 0u && lw.elem[rw] + (kw - lw.pos[rw]) == keep;
+                    --kw;
+                }
+                good = good && hit >= 0;
+                pos = lw.elem[rw] + (kw - lw.pos[rw]);
+                item = lw.item[rw] + (kw - lw.pos[rw]);
+            }
+        } else if (!(choice <= 0.0f)) {
+            good = false;
+        }
+        if (lane == 0) {
+            sh.ok = good ? 1u : 0u;
+            sh.keep = keep;
+            sh.pos = pos;
+            sh.item = item;
+            sh.s = static_cast<double>(choice);
+            sh.token = -1;
+        }
     }
     __syncthreads();
-    // Whether every item before `last` that stands for a bin was passed in the
-    // binade the plan took it in (tag bits 0-7 for the cumulative, 8-15 for the
-    // walk), and no event fell on one.
-    auto check = [&](int n_log, int last, uint32_t first_expo, int shift) {
-        __syncthreads();  // the log is written
-        if (n_log > kDrawLog && tid == 0) sh.bad = 1u;
-        const int n = min(n_log, kDrawLog);
-        for (int i = tid; i < last; i += kDrawThreads) {
-            const uint64_t it = items[i];
-            if (!(it & kFbRegular)) continue;
-            uint32_t e = first_expo;
-            bool hit = false;
-            for (int l = 0; l < n; ++l) {
-                const int li = sh.log_item[l];
-                if (li < i) e = sh.log_expo[l];
-                hit = hit || li == i;
+    ok = ok && sh.ok != 0u;
+    const uint32_t pos = sh.pos, keep = sh.keep;
+    const int item = static_cast<int>(sh.item);
+    bool near = false;
+    if (ok) {
+        // Near-boundary flag: double sums of the probabilities before and
+        // through the chosen position; the sum before the draw's bins is
+        // fb_collect's, the rest its single tokens.
+        const double ch = sh.s;
+        double before = 0.0;
+        bool nb = false, na = false;
+        if (pos > 0u) {
+            if (item < draw0 || item >= draw1) {
+                ok = false;
+            } else {
+                double t = 0.0;
+                for (int i = draw0 + tid; i < item; i += kThreads)
+                    t += static_cast<double>(u2f(static_cast<uint32_t>(items[i] >> 32)) * inv);
+                t = wave::sum_f64(t);
+                if (lane == 0) sh.sd[wave] = t;
+                __syncthreads();
+                before = wave::sum_f64(lane < parts ? r.pbef[lane] : 0.0);
+                for (int v = 0; v < kWaves; ++v) before += sh.sd[v];
+                ok = near_decided(ch, before, near_sum_error(pos), nb);
             }
-            if (hit || ((static_cast<uint32_t>(it) >> shift) & 0xffu) != e) sh.bad = 1u;
         }
-        __syncthreads();
-    };
-    auto expanded = [&](int i) { return i >= 0 && i < G && !(items[i] & kFbRegular); };
-    uint32_t pos = 0;
-    int item = 0;
-    bool ok = true, near = false;
-    {
-        double s = static_cast<double>(q0);
-        ChainPos cp{0, 1};
-        uint32_t keep = keff;
-        if (keff > 1u) {
-            const uint32_t L = min(keff, end);
-            DrawLog log{&sh};
-            const bool hit = L > 1u && bchain::block_chain<bchain::F32Acc, false, kDrawThreads>(
-                                           pre, aux, inv, G, cp, L, s, static_cast<double>(p.top_p), sh.bc, log);
-            if (hit) keep = cp.elem + 1u;
-            else if (L < keff) ok = false;  // the plan's items end before the cut
-            check(log.n, min(cp.item + 1, G), static_cast<uint32_t>(fb_expo(static_cast<double>(q0))), 0);
-        }
-        const float mass = static_cast<float>(s);
-        const float u = a.uniforms[row];
-        const float choice = u * (mass - 0.0f) + 0.0f;  // random.h:1864-1871
-        if (ok && choice > 0.0f && choice < __builtin_inff()) {
-            ChainPos w{0, 0};
-            double c = static_cast<double>(choice);
-            DrawLog log{&sh};
-            const bool stop = bchain::block_chain<bchain::F32Acc, true, kDrawThreads>(pre, aux, inv, G, w, min(keep, end), c,
-                                                                                     0.0, sh.bc, log);
-            pos = stop ? w.elem : keep - 1u;
-            item = w.item;
-            check(log.n, min(item + 1, G), static_cast<uint32_t>(fb_expo(static_cast<double>(choice))), 8);
-        } else if (!(choice <= 0.0f)) {
-            ok = false;
-        }
-        ok = ok && expanded(item) && sh.bad == 0u;
-        if (ok) {
-            // Near-boundary flag: double sums of the probabilities before and
-            // through the chosen position; the sum before the draw's bins is
-            // fb_collect's, the rest its single tokens.
-            double before = 0.0;
-            bool nb = false, na = false;
-            const double ch = static_cast<double>(choice);
-            bool sure = true;
-            if (pos > 0u) {
-                if (item < draw0 || item >= draw1) {
-                    sure = false;
-                } else {
-                    double t = 0.0;
-                    for (int i = draw0 + tid; i < item; i += kDrawThreads) t += static_cast<double>(aux[i] * inv);
-                    t = wave::sum_f64(t);
-                    if (lane == 0) sh.sums[wave] = t;
-                    __syncthreads();
-                    before = wave::sum_f64(lane < parts ? r.pbef[lane] : 0.0);
-                    for (int v = 0; v < kDrawWaves; ++v) before += sh.sums[v];
-                    sure = near_decided(ch, before, near_sum_error(pos), nb);
-                }
-            }
-            sure = sure && near_decided(ch, before + static_cast<double>(aux[item] * inv), near_sum_error(pos), na);
-            near = (pos > 0u && nb) || (pos + 1u < keep && na);
-            ok = sure;
-        }
+        const float q = u2f(static_cast<uint32_t>(items[item] >> 32)) * inv;
+        ok = ok && near_decided(ch, before + static_cast<double>(q), near_sum_error(pos), na);
+        near = (pos > 0u && nb) || (pos + 1u < keep && na);
     }
     if (!ok) {  // block-uniform
         if (tid == 0) meta[kMetaStatus] = kStatusToSort;
@@ -889,6 +1169,8 @@ __global__ __launch_bounds__(kDrawThreads) void fb_draw_kernel(DevArgs a, int pa
     uint32_t* bitmap = a.fo_bitmap + static_cast<int64_t>(row) * a.fo_bitmap_words;
     const float* rowp = static_cast<const float*>(a.logits) + static_cast<int64_t>(row) * a.row_stride;
     const uint32_t peb = static_cast<uint32_t>(items[item] >> 32);
+    const int G = static_cast<int>(meta[kMetaItems]);
+    // (the tokens of one exp lie in one bin; bins beside it hold other exps)
     auto same = [&](int i) { return i >= 0 && i < G && static_cast<uint32_t>(items[i] >> 32) == peb; };
     int is = item, ie = item;  // (every wave finds the same run)
     for (;;) {
@@ -904,21 +1186,22 @@ __global__ __launch_bounds__(kDrawThreads) void fb_draw_kernel(DevArgs a, int pa
         if (n < 64) break;
     }
     const int n_tie = ie - is + 1;
+    uint64_t* tie = sh.list[0].tie;
     if (n_tie == 1) {
         if (tid == 0) sh.token = static_cast<int32_t>(composite_index(items[item]));
     } else {  // (at most kFbSegMost: one exp lies in one bin)
-        for (int i = tid; i < n_tie; i += kDrawThreads) {
+        for (int i = tid; i < n_tie; i += kThreads) {
             const uint32_t idx = composite_index(items[is + i]);
             float v = softcap(rowp[idx], p.softcap);
             if (pen && ((bitmap[idx >> 5] >> (idx & 31u)) & 1u)) v = penalize(v, p.repetition_penalty);
-            sh.tie[i] = composite(order_key(v), idx);
+            tie[i] = composite(order_key(v), idx);
         }
         __syncthreads();
         const uint32_t want = static_cast<uint32_t>(item - is);
-        for (int i = tid; i < n_tie; i += kDrawThreads) {
-            const uint64_t x = sh.tie[i];
+        for (int i = tid; i < n_tie; i += kThreads) {
+            const uint64_t x = tie[i];
             uint32_t rank = 0;
-            for (int j = 0; j < n_tie; ++j) rank += sh.tie[j] > x ? 1u : 0u;
+            for (int j = 0; j < n_tie; ++j) rank += tie[j] > x ? 1u : 0u;
             if (rank == want) sh.token = static_cast<int32_t>(composite_index(x));
         }
     }
@@ -926,13 +1209,44 @@ __global__ __launch_bounds__(kDrawThreads) void fb_draw_kernel(DevArgs a, int pa
     // The bitmap is all zero again after every call (cleared from the history
     // before the token is appended: a full ring's history is the ring).
     if (pen) {
-        for (int i = tid; i < H; i += kDrawThreads) {
+        for (int i = tid; i < H; i += kThreads) {
             const int32_t id = hist[i];
             if (id >= 0 && id < V) bitmap[id >> 5] = 0u;
         }
         __syncthreads();
     }
-    if (tid == 0) emit_row(a, row, sh.token, aux[item] * inv, near ? GE_FLAG_NEAR_BOUNDARY : 0);
+    if (tid == 0) emit_row(a, row, sh.token, u2f(peb) * inv, near ? GE_FLAG_NEAR_BOUNDARY : 0);
+}
+
+// ---- launches ----------------------------------------------------------------
+
+constexpr int kOT = 256;  // threads of fb_order_kernel
+constexpr int kDT = 512;  // and of fb_draw_kernel
+
+__global__ __launch_bounds__(kFT) void fb_range_kernel(DevArgs a) {
+    __shared__ RangeShared sh;
+    fb_range(a, blockIdx.y, blockIdx.x, gridDim.x, sh);
+}
+__global__ __launch_bounds__(kFT) void fb_exps_kernel(DevArgs a) {
+    __shared__ ExpsShared sh;
+    fb_exps(a, blockIdx.y, blockIdx.x, gridDim.x, sh);
+}
+template <int kPer>
+__global__ __launch_bounds__(kFT) void fb_plan_kernel(DevArgs a, int parts) {
+    __shared__ PlanShared sh;
+    fb_plan<kPer>(a, blockIdx.x, parts, sh);
+}
+__global__ __launch_bounds__(kFT) void fb_collect_kernel(DevArgs a) {
+    __shared__ CollectShared sh;
+    fb_collect(a, blockIdx.y, blockIdx.x, gridDim.x, sh);
+}
+__global__ __launch_bounds__(kOT) void fb_order_kernel(DevArgs a) {
+    __shared__ OrderShared sh;
+    fb_order<kOT>(a, blockIdx.y, blockIdx.x, gridDim.x, sh);
+}
+__global__ __launch_bounds__(kDT) void fb_draw_kernel(DevArgs a, int parts) {
+    __shared__ DrawShared sh;
+    fb_draw<kDT>(a, blockIdx.x, parts, sh);
 }
 
 }  // namespace
@@ -952,10 +1266,13 @@ hipError_t launch_binned(const DevArgs& a, hipStream_t stream) {
         case 8: hipLaunchKernelGGL(fb_plan_kernel<8>, rows, dim3(kFT), 0, stream, a, parts); break;
         default: hipLaunchKernelGGL(fb_plan_kernel<16>, rows, dim3(kFT), 0, stream, a, parts); break;
     }
-    hipLaunchKernelGGL(fb_collect_kernel, grid, dim3(kFT), 0, stream, a);
+    // (one part for many rows: its places need no counting pass)
+    const int cparts = a.rows >= 128 ? 1 : parts;
+    hipLaunchKernelGGL(fb_collect_kernel, dim3(static_cast<unsigned>(cparts), static_cast<unsigned>(a.rows)), dim3(kFT), 0,
+                       stream, a);
     const unsigned ob = static_cast<unsigned>(std::max(4, std::min(128, 2048 / a.rows)));
     hipLaunchKernelGGL(fb_order_kernel, dim3(ob, static_cast<unsigned>(a.rows)), dim3(kOT), 0, stream, a);
-    hipLaunchKernelGGL(fb_draw_kernel, rows, dim3(kDrawThreads), 0, stream, a, parts);
+    hipLaunchKernelGGL(fb_draw_kernel, rows, dim3(kDT), 0, stream, a, cparts);
     return hipGetLastError();
 }
 

@@ -115,11 +115,12 @@ constexpr int64_t fo_tile_words(int tiles) { return static_cast<int64_t>(tiles) 
 constexpr int kFbMaxBins = 16384;
 constexpr int kFbParts = 64;    // workgroups that stream one row, at most
 constexpr int kFbSegs = 4096;   // expanded bins of one row, at most
+constexpr int kFbSegWords = 10; // words of one's record
 __host__ __device__ constexpr int fb_bins(int vocab) {
     return vocab >= 131072 ? kFbMaxBins : vocab >= 65536 ? kFbMaxBins / 2 : vocab >= 32768 ? kFbMaxBins / 4 : kFbMaxBins / 8;
 }
 __host__ __device__ constexpr int64_t fb_row_words(int vocab) {
-    return fb_bins(vocab) + 6 * kFbParts + 64 + kFbMaxBins / 32 + 3 * kFbSegs;
+    return fb_bins(vocab) + 6 * kFbParts + 64 + kFbMaxBins / 32 + kFbSegWords * (kFbSegs + 2);
 }
 
 // The row's parameters: the shared ones, or its entry of row_params.
