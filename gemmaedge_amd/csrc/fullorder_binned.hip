@@ -157,6 +157,36 @@ __device__ __forceinline__ void fb_stream(const float* rowp, bool vec, int lo, i
     }
 }
 
+// f(first token, x[kU][4], tokens from it on): one call per step of kU 16-byte
+// loads per thread, load u at first + u * kFStep; the last step may be partial
+// (tokens past the end repeat the last one).
+template <int kU, typename F>
+__device__ __forceinline__ void fb_stream_steps(const float* rowp, bool vec, int lo, int hi, int tid, F&& f) {
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    for (int base = lo; base < hi; base += kU * kFStep) {
+        float x[kU][4];
+        const int i0 = base + tid * 4;
+        if (vec && base + kU * kFStep <= hi) {
+            v4 q[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) q[u] = *reinterpret_cast<const v4*>(rowp + i0 + u * kFStep);
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                x[u][0] = q[u].x;
+                x[u][1] = q[u].y;
+                x[u][2] = q[u].z;
+                x[u][3] = q[u].w;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[u][j] = rowp[min(i0 + u * kFStep + j, hi - 1)];
+        }
+        f(i0, x, base + kU * kFStep <= hi ? kU * kFStep : hi - i0);
+    }
+}
+
 // Largest and smallest of one key per thread over the workgroup.
 __device__ __forceinline__ uint32_t fb_block_max(uint32_t v, uint32_t* s) {
     const uint32_t w = wave::max_u32(v);
@@ -287,34 +317,58 @@ __device__ __forceinline__ void fb_exps(const DevArgs& a, int row, int part, int
     const uint32_t* bitmap = a.fo_bitmap + static_cast<int64_t>(row) * a.fo_bitmap_words;
     float* pes = fb_exp_array(a, row);
     const float inv_temp = 1.0f / p.temperature;
+    const float cap = p.softcap;
+    // The narrow softcaps apply to a step whose logits all lie in their range
+    // (one vote per 16 tokens a lane). Below 2^-100 * cap the quotients may round
+    // otherwise, which no exp shows unless 1 / T is huge.
+    const bool capped = cap > 0.0f;
+    const bool narrow = capped && cap >= 0x1p-60f && cap <= 0x1p60f && inv_temp <= 0x1p40f;
+    const float small = narrow ? cap * kSoftcapSmall : -1.0f, below = narrow ? cap * kSoftcapBelowOne : -1.0f;
+    const float yc = narrow ? recip_step(cap) : 0.0f;
     double sum = 0.0;
-    fb_stream<4>(rowp, a.vec_ok != 0, lo, hi, tid, [&](int i, float x0, float x1, float x2, float x3, int n) {
-        const uint32_t bits = pen && n ? bitmap[i >> 5] >> (i & 31) : 0u;
-        const float x[4] = {x0, x1, x2, x3};
-        float pe[4];
+    fb_stream_steps<4>(rowp, a.vec_ok != 0, lo, hi, tid, [&](int i0, const float (&x)[4][4], int n) {
+        float most = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float v = softcap(x[j], p.softcap);
-            if ((bits >> j) & 1u) v = penalize(v, p.repetition_penalty);
-            pe[j] = expf_glibc_tab((v - vmax) * inv_temp, [&](uint32_t t) { return tab[t]; });
-        }
-        if (n == 4) {
-            *reinterpret_cast<float4*>(pes + i) = make_float4(pe[0], pe[1], pe[2], pe[3]);
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                sum += static_cast<double>(pe[j]);
-                atomicAdd(&hist_s[fb_bin(pe[j], shift, static_cast<uint32_t>(bins))], 1u);
-            }
-        } else {
+            for (int j = 0; j < 4; ++j) most = fmaxf(most, __builtin_fabsf(x[u][j]));
+        auto take = [&](auto&& cap_of) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (j < n) {
-                    pes[i + j] = pe[j];
-                    sum += static_cast<double>(pe[j]);
-                    atomicAdd(&hist_s[fb_bin(pe[j], shift, static_cast<uint32_t>(bins))], 1u);
+            for (int u = 0; u < 4; ++u) {
+                const int i = i0 + u * kFStep;
+                const int nu = min(max(n - u * kFStep, 0), 4);
+                if (n < 4 * kFStep && nu == 0) continue;
+                const uint32_t bits = pen ? bitmap[i >> 5] >> (i & 31) : 0u;
+                float pe[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float v = cap_of(x[u][j]);
+                    if ((bits >> j) & 1u) v = penalize(v, p.repetition_penalty);
+                    pe[j] = expf_glibc_tab((v - vmax) * inv_temp, [&](uint32_t t) { return tab[t]; });
+                }
+                if (n >= 4 * kFStep || nu == 4) {
+                    *reinterpret_cast<float4*>(pes + i) = make_float4(pe[0], pe[1], pe[2], pe[3]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        sum += static_cast<double>(pe[j]);
+                        atomicAdd(&hist_s[fb_bin(pe[j], shift, static_cast<uint32_t>(bins))], 1u);
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        if (j < nu) {
+                            pes[i + j] = pe[j];
+                            sum += static_cast<double>(pe[j]);
+                            atomicAdd(&hist_s[fb_bin(pe[j], shift, static_cast<uint32_t>(bins))], 1u);
+                        }
+                    }
                 }
             }
-        }
+        };
+        if (!capped) take([&](float v) { return v; });
+        else if (__ballot(!(most <= small)) == 0ull) take([&](float v) { return softcap_range<kSoftcapRangeSmall>(v, cap, yc); });
+        else if (__ballot(!(most <= below)) == 0ull) take([&](float v) { return softcap_range<kSoftcapRangeBelowOne>(v, cap, yc); });
+        else take([&](float v) { return softcap(v, cap); });
     });
     sum = wave::sum_f64(sum);
     if ((tid & 63) == 0) sums[tid >> 6] = sum;

@@ -276,6 +276,76 @@ __host__ __device__ inline float softcap(float l, float c) {
     return (c > 0.0f) ? c * tanhf_fdlibm(l / c) : l;
 }
 
+#if defined(__HIPCC__)
+// ---- softcap over narrow ranges (device) -------------------------------------
+//
+// The same operations as softcap(), without the cases that cannot occur: over
+// kSmall, |l| <= kSoftcapSmall * c, expm1's argument lies within ln2 / 2, where
+// its reduction is the identity; over kBelowOne, |l| <= kSoftcapBelowOne * c,
+// tanh takes its |x| < 1 form and expm1's argument is negative. Divisions run
+// the hardware's own sequence (v_rcp_f32, one Newton step, the quotient and two
+// corrections) without its scaling of extreme operands, which a divisor and a
+// dividend above 2^-100 do not need: the results are those of softcap() for
+// |l| = 0 (without its sign) and |l| >= 2^-100 * c, and 2^-100 <= c <= 2^100.
+// tests/test_gpu_softcap_ranges.py compares both on every such float.
+constexpr float kSoftcapSmall = 0.173f;
+constexpr float kSoftcapBelowOne = 0.999f;
+enum SoftcapRange { kSoftcapAny = 0, kSoftcapRangeBelowOne = 1, kSoftcapRangeSmall = 2 };
+
+__device__ inline float recip_step(float b) {  // 1 / b, one Newton step on v_rcp_f32
+    const float y = __builtin_amdgcn_rcpf(b);
+    return fmaf(fmaf(-b, y, 1.0f), y, y);
+}
+__device__ inline float quotient(float a, float b, float y) {  // a / b, y = recip_step(b)
+    const float q0 = a * y;
+    const float q1 = fmaf(fmaf(-b, q0, a), y, q0);
+    return fmaf(fmaf(-b, q1, a), y, q1);
+}
+
+template <int kRange>
+__device__ inline float softcap_range(float l, float c, float yc) {  // yc = recip_step(c)
+    static_assert(kRange == kSoftcapRangeBelowOne || kRange == kSoftcapRangeSmall, "a narrow range");
+    const float ln2_hi = u2f(0x3f317180u);
+    const float ln2_lo = u2f(0x3717f7d1u);
+    const float invln2 = u2f(0x3fb8aa3bu);
+    const float Q1 = u2f(0xbd088889u), Q2 = u2f(0x3ad00d01u), Q3 = u2f(0xb8a670cdu),
+                Q4 = u2f(0x36867e54u), Q5 = u2f(0xb457edbbu);
+    const float z0 = quotient(l, c, yc);
+    const float y = -2.0f * __builtin_fabsf(z0);  // expm1's argument
+    float x = y, cc = 0.0f;
+    int32_t k = 0;
+    if constexpr (kRange == kSoftcapRangeBelowOne) {
+        const uint32_t hx = f2u(y) & 0x7fffffffu;
+        const int32_t kg = static_cast<int32_t>(invln2 * y - 0.5f);
+        k = hx <= 0x3eb17218u ? 0 : (hx < 0x3F851592u ? -1 : kg);
+        const float t = static_cast<float>(k);
+        const float hi = y - t * ln2_hi;
+        const float lo = t * ln2_lo;
+        x = hi - lo;
+        cc = (hi - x) - lo;
+    }
+    const float hfx = 0.5f * x;
+    const float hxs = x * hfx;
+    const float r1 = 1.0f + hxs * (Q1 + hxs * (Q2 + hxs * (Q3 + hxs * (Q4 + hxs * Q5))));
+    const float tt = 3.0f - r1 * hfx;
+    const float d = 6.0f - x * tt;
+    const float e0 = hxs * quotient(r1 - tt, d, recip_step(d));
+    float t = x - (x * e0 - hxs);  // k == 0
+    if constexpr (kRange == kSoftcapRangeBelowOne) {
+        const float e = (x * (e0 - cc) - cc) - hxs;
+        const float resm1 = 0.5f * (x - e) - 0.5f;                                                 // k == -1
+        const float yb = u2f(f2u(1.0f - (e - x)) + (static_cast<uint32_t>(k) << 23)) - 1.0f;      // k <= -2
+        t = k == 0 ? t : (k == -1 ? resm1 : yb);
+    }
+    t = (f2u(y) & 0x7fffffffu) < 0x33000000u ? y : t;  // |y| < 2^-25
+    const float b = t + 2.0f;
+    float z = quotient(-t, b, recip_step(b));
+    z = __builtin_copysignf(z, z0);
+    if ((f2u(z0) & 0x7fffffffu) < 0x24000000u) z = z0 * (1.0f + z0);  // |x| < 2^-55
+    return c * z;
+}
+#endif
+
 // Repetition penalty (CTRL rule): v > 0 ? v / r : v * r.
 __host__ __device__ inline float penalize(float v, float r) { return v > 0.0f ? v / r : v * r; }
 

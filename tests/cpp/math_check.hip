@@ -59,7 +59,39 @@ __global__ void digest_kernel(int fn, uint64_t* out) {
                                     static_cast<unsigned long long>(red[0]));
 }
 
+// Inputs of a narrow softcap's range for which it differs from softcap().
+template <int kRange>
+__global__ void range_kernel(float c, float most, unsigned long long* out) {
+    const uint64_t base = static_cast<uint64_t>(blockIdx.x) << 16;
+    const float yc = ge::recip_step(c);
+    unsigned long long bad = 0;
+    for (int i = 0; i < 256; ++i) {
+        const float l = ge::u2f(static_cast<uint32_t>(base + static_cast<uint64_t>(i) * 256u + threadIdx.x));
+        const float m = __builtin_fabsf(l);
+        if (!(m <= most) || (m != 0.0f && m < 0x1p-100f * c)) continue;
+        const float want = ge::softcap(l, c), got = ge::softcap_range<kRange>(l, c, yc);
+        if (want == 0.0f ? got != 0.0f : ge::f2u(want) != ge::f2u(got)) ++bad;
+    }
+    if (bad) atomicAdd(out, bad);
+}
+
 }  // namespace
+
+// range 1: below one, 2: small (ge_math.h). Negative: a HIP error.
+extern "C" long long ge_test_softcap_range_mismatches(int range, float c) {
+    unsigned long long* d = nullptr;
+    unsigned long long h = 0;
+    if (hipMalloc(&d, sizeof(h)) != hipSuccess) return -1;
+    if (hipMemcpy(d, &h, sizeof(h), hipMemcpyHostToDevice) != hipSuccess) return -1;
+    if (range == ge::kSoftcapRangeSmall)
+        hipLaunchKernelGGL(range_kernel<ge::kSoftcapRangeSmall>, dim3(65536), dim3(256), 0, 0, c, c * ge::kSoftcapSmall, d);
+    else
+        hipLaunchKernelGGL(range_kernel<ge::kSoftcapRangeBelowOne>, dim3(65536), dim3(256), 0, 0, c,
+                           c * ge::kSoftcapBelowOne, d);
+    const hipError_t e = hipMemcpy(&h, d, sizeof(h), hipMemcpyDeviceToHost);
+    (void)hipFree(d);
+    return e == hipSuccess ? static_cast<long long>(h) : -1;
+}
 
 extern "C" long long ge_test_host_mismatches(int fn, uint32_t lo, uint64_t count, int nthreads) {
     std::atomic<long long> bad{0};
