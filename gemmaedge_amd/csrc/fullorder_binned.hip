@@ -207,7 +207,7 @@ __device__ __forceinline__ void fb_range(const DevArgs& a, int row, int part, in
     uint32_t* s = sh.s;
     const int tid = threadIdx.x;
     ge_sample_params p;
-    const int bins = fb_bins(a.vocab);
+    const int bins = a.fo_bins;
     if (!fb_serves(a, row, p)) {
         uint32_t k;
         // (a row of this pass that the sort-based one serves: 1024 < k < V)
@@ -291,7 +291,7 @@ __device__ __forceinline__ void fb_exps(const DevArgs& a, int row, int part, int
     const int tid = threadIdx.x;
     ge_sample_params p;
     if (!fb_serves(a, row, p)) return;
-    const int bins = fb_bins(a.vocab);
+    const int bins = a.fo_bins;
     const FbRow r = fb_row(a, row, bins);
     if (tid < 64) {
         float vm;
@@ -378,10 +378,12 @@ __device__ __forceinline__ void fb_exps(const DevArgs& a, int row, int part, int
         for (int w = 0; w < kFW; ++w) t += sums[w];
         r.psum[part] = t;
     }
-    for (int i = tid; i < bins; i += kFT) {
-        const uint32_t c = hist_s[i];
-        if (parts == 1) r.bin[i] = c;
-        else if (c) atomicAdd(&r.bin[i], c);
+    // (two bins per word: the counts do not reach 2^32)
+    unsigned long long* out = reinterpret_cast<unsigned long long*>(r.bin);
+    for (int i = tid; i < bins / 2; i += kFT) {
+        const unsigned long long c = (static_cast<unsigned long long>(hist_s[2 * i + 1]) << 32) | hist_s[2 * i];
+        if (parts == 1) out[i] = c;
+        else if (c) atomicAdd(&out[i], c);
     }
 }
 
@@ -395,6 +397,7 @@ __device__ __forceinline__ double fb_scan_f64(double v, double* s, double& total
     __syncthreads();
     double before = 0.0;
     total = 0.0;
+#pragma unroll
     for (int w = 0; w < kWaves; ++w) {
         if (w == wave) before = total;
         total += s[w];
@@ -402,20 +405,39 @@ __device__ __forceinline__ double fb_scan_f64(double v, double* s, double& total
     __syncthreads();
     return before + (incl - v);
 }
+// The same for two counts and a double at once: v, w and x become their
+// exclusive prefixes.
 template <int kWaves>
-__device__ __forceinline__ uint32_t fb_scan_u32(uint32_t v, uint32_t* s, uint32_t& total) {
+__device__ __forceinline__ void fb_scan_3(uint32_t& v, uint32_t& w, double& x, double* sx, uint32_t* sv, uint32_t* sw,
+                                          uint32_t& v_all, uint32_t& w_all, double& x_all) {
     const int wave = threadIdx.x >> 6;
-    const uint32_t incl = wave::incl_add(v);
-    if ((threadIdx.x & 63) == 63) s[wave] = incl;
-    __syncthreads();
-    uint32_t before = 0;
-    total = 0;
-    for (int w = 0; w < kWaves; ++w) {
-        if (w == wave) before = total;
-        total += s[w];
+    const uint32_t iv = wave::incl_add(v), iw = wave::incl_add(w);
+    const double ix = wave::incl_f64(x);
+    if ((threadIdx.x & 63) == 63) {
+        sv[wave] = iv;
+        sw[wave] = iw;
+        sx[wave] = ix;
     }
     __syncthreads();
-    return before + incl - v;
+    uint32_t bv = 0, bw = 0;
+    double bx = 0.0;
+    v_all = w_all = 0;
+    x_all = 0.0;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+        if (i == wave) {
+            bv = v_all;
+            bw = w_all;
+            bx = x_all;
+        }
+        v_all += sv[i];
+        w_all += sw[i];
+        x_all += sx[i];
+    }
+    __syncthreads();
+    v = bv + iv - v;
+    w = bw + iw - w;
+    x = bx + (ix - x);
 }
 
 // The biased float exponent of x > 0, at least 1 (subnormal floats share the
@@ -442,7 +464,7 @@ struct PlanShared {
     uint32_t c[kFbMaxBins + kFbMaxBins / 16];  // counts (padded: a thread's bins lie 17 words from the next's)
     uint32_t w[kFbMaxBins + kFbMaxBins / 16];  // the bin's rounded sum (a float), then what it is
     double sd[kFW];
-    uint32_t su[kFW];
+    uint32_t su[kFW], sv[kFW];
     uint32_t mask[kFbMaxBins / 32];
     uint32_t bad, cut, stop, first, last, off0, off1;
     double cut_lo, cut_hi;
@@ -509,9 +531,11 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
         t += static_cast<double>(static_cast<float>(c) * mid(b));
     });
     if (low != 0xffffffffu) atomicMin(&sh.cut, low);
-    uint32_t total, n_fine;
-    const uint32_t before = fb_scan_u32<kFW>(n_t, sh.su, total);  // elements before this thread's bins
-    (void)fb_scan_u32<kFW>(fine, sh.su, n_fine);
+    // one scan for the elements before this thread's bins, the fine terms' number
+    // and the exact sum (x)
+    uint32_t before = n_t, n_f = fine, total, n_fine;
+    double x = t, all;
+    fb_scan_3<kFW>(before, n_f, x, sh.sd, sh.su, sh.sv, total, n_fine, all);
     const float inv_temp = 1.0f / p.temperature;
     const bool fits = inv_temp > 0.0f && inv_temp < __builtin_inff() && vmax > -__builtin_inff() &&
                       vmax < __builtin_inff() && total == static_cast<uint32_t>(V) && den_rounds_alike(S, n_fine, V);
@@ -523,8 +547,6 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
     // then with every addend rounded as it is there (A). The bins' middles miss
     // the exact sum mostly where few large addends hold most of it, in the head
     // (always replayed): the bins after it begin that much later.
-    double all;
-    double x = fb_scan_f64<kFW>(t, sh.sd, all);
     const double corr = S * static_cast<double>(inv) - all;
     x += corr;
     t = 0.0;
@@ -634,12 +656,11 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
         W = W1;
     });
     uint32_t G, segs, elems;
-    uint32_t off = fb_scan_u32<kFW>(n_items, sh.su, G);
-    uint32_t seg = fb_scan_u32<kFW>(n_seg, sh.su, segs);
-    (void)fb_scan_u32<kFW>(n_elem, sh.su, elems);
     double cum_all, walk_all;
-    double cum = fb_scan_f64<kFW>(s_cum, sh.sd, cum_all);
-    double walk = fb_scan_f64<kFW>(s_walk, sh.sd, walk_all);
+    double cum = s_cum, walk = s_walk;
+    uint32_t off = n_items, seg = n_seg, elems_at = n_elem, unused = 0, none_all;
+    fb_scan_3<kFW>(off, seg, cum, sh.sd, sh.su, sh.sv, G, segs, cum_all);
+    fb_scan_3<kFW>(elems_at, unused, walk, sh.sd, sh.su, sh.sv, elems, none_all, walk_all);
     if (sh.bad || static_cast<int64_t>(G) + 1 > fb_half(a) || segs > static_cast<uint32_t>(kFbSegs)) {
         if (tid == 0) meta[kMetaStatus] = kStatusToSort;
         return;
@@ -701,7 +722,7 @@ __device__ __forceinline__ void fb_collect(const DevArgs& a, int row, int part, 
     const int tid = threadIdx.x;
     ge_sample_params p;
     if (!fb_serves(a, row, p) || fb_meta(a, row)[kMetaStatus] != kStatusOk) return;
-    const int bins = fb_bins(a.vocab);
+    const int bins = a.fo_bins;
     const FbRow r = fb_row(a, row, bins);
     for (int i = tid; i < bins / 32; i += kFT) sh.mask[i] = r.mask[i];
     for (int i = tid; i < bins; i += kFT) sh.next[i] = parts == 1 ? r.bin[i] : 0u;
@@ -772,7 +793,7 @@ __device__ __forceinline__ void fb_order(const DevArgs& a, int row, int block, i
     ge_sample_params p;
     uint32_t* meta = fb_meta(a, row);
     if (!fb_serves(a, row, p) || meta[kMetaStatus] != kStatusOk) return;
-    const FbRow r = fb_row(a, row, fb_bins(a.vocab));
+    const FbRow r = fb_row(a, row, a.fo_bins);
     const int segs = static_cast<int>(r.scal[kScSegs]);
     const float inv = u2f(r.scal[kScInv]);
     uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
@@ -924,8 +945,8 @@ struct DrawList {
 static_assert(kDrawList * 4 == kDrawTies * 8, "the union");
 struct DrawShared {
     DrawList list[2];  // cumulative, walk
-    double sd[16];
-    uint32_t su[16], sr[16];
+    double sd[32];
+    uint32_t su[32], sr[32];
     double s;
     uint32_t keep, pos, item, near_u, ok;
     int32_t token;
@@ -980,27 +1001,27 @@ __device__ __forceinline__ bool draw_lists(const FbRow& r, int segs, const uint6
         const double ti = wave::incl_f64(t[x]);
         const uint32_t ni = wave::incl_add(n[x]), ri = wave::incl_add(at[x]);
         if ((tid & 63) == 63) {
-            sh.sd[8 * x + wave] = ti;
-            sh.su[8 * x + wave] = ni;
-            sh.sr[8 * x + wave] = ri;
+            sh.sd[16 * x + wave] = ti;
+            sh.su[16 * x + wave] = ni;
+            sh.sr[16 * x + wave] = ri;
         }
         t[x] = ti - t[x];
         n[x] = ni - n[x];
         at[x] = ri - at[x];
     }
-    static_assert(kWaves <= 8, "the scan's words");
+    static_assert(kWaves <= 16, "the scan's words");
     __syncthreads();
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
         n_all[x] = r_all[x] = 0;
         for (int w = 0; w < kWaves; ++w) {
             if (w < wave) {
-                t[x] += sh.sd[8 * x + w];
-                n[x] += sh.su[8 * x + w];
-                at[x] += sh.sr[8 * x + w];
+                t[x] += sh.sd[16 * x + w];
+                n[x] += sh.su[16 * x + w];
+                at[x] += sh.sr[16 * x + w];
             }
-            n_all[x] += sh.su[8 * x + w];
-            r_all[x] += sh.sr[8 * x + w];
+            n_all[x] += sh.su[16 * x + w];
+            r_all[x] += sh.sr[16 * x + w];
         }
     }
     if (max(n_all[0], n_all[1]) > static_cast<uint32_t>(kDrawList) || max(r_all[0], r_all[1]) > static_cast<uint32_t>(kDrawRegions))
@@ -1114,7 +1135,7 @@ __device__ __forceinline__ void fb_draw(const DevArgs& a, int row, int parts, Dr
     uint32_t* meta = fb_meta(a, row);
     if (meta[kMetaStatus] != kStatusOk) return;  // the sort-based pass serves the row
     const int V = a.vocab;
-    const FbRow r = fb_row(a, row, fb_bins(V));
+    const FbRow r = fb_row(a, row, a.fo_bins);
     const int segs = static_cast<int>(r.scal[kScSegs]);
     const uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
     const float inv = u2f(r.scal[kScInv]);
@@ -1303,14 +1324,69 @@ __global__ __launch_bounds__(kDT) void fb_draw_kernel(DevArgs a, int parts) {
     fb_draw<kDT>(a, blockIdx.x, parts, sh);
 }
 
+// Calls with per-row parameters: one workgroup takes a row through every stage.
+// The host cannot tell whether any row needs this path, and six launches cost
+// 20 us when none does; a served row takes longer than spread over the chip (its
+// exps run on one CU), but many rows run side by side.
+union RowShared {
+    RangeShared range;
+    ExpsShared exps;
+    PlanShared plan;
+    CollectShared collect;
+    OrderShared order;
+    DrawShared draw;
+    __device__ RowShared() {}
+};
+// The stage's stores and atomics done and seen by the workgroup's loads (some
+// were made in L2, past the CU's L1).
+__device__ __forceinline__ void stage_done() {
+    __threadfence();
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+}
+template <int kPer>
+__global__ __launch_bounds__(kFT) void fb_row_kernel(DevArgs a) {
+    __shared__ RowShared sh;
+    const int row = blockIdx.x;
+    ge_sample_params p;
+    uint32_t k;
+    fb_range(a, row, 0, 1, sh.range);
+    if (!fb_serves(a, row, p)) {  // (block-uniform) done rows are reported by the draw
+        if (full_order_row(p, a.vocab, k) && row_done(a, row)) fb_draw<kFT>(a, row, 1, sh.draw);
+        return;
+    }
+    stage_done();
+    fb_exps(a, row, 0, 1, sh.exps);
+    stage_done();
+    fb_plan<kPer>(a, row, 1, sh.plan);
+    stage_done();
+    fb_collect(a, row, 0, 1, sh.collect);
+    stage_done();
+    fb_order<kFT>(a, row, 0, 1, sh.order);
+    stage_done();
+    fb_draw<kFT>(a, row, 1, sh.draw);
+}
+
 }  // namespace
 
-hipError_t launch_binned(const DevArgs& a, hipStream_t stream) {
+hipError_t launch_binned(const DevArgs& args, hipStream_t stream) {
+    DevArgs a = args;
+    a.fo_bins = fb_bins(a.vocab, a.rows);
     // Parts per row: about two workgroups per CU in all, at most one per step.
     const int steps = (a.vocab + kFStep - 1) / kFStep;
     const int parts = std::max(1, std::min({steps, kFbParts, (512 + a.rows - 1) / a.rows}));
     const dim3 grid(static_cast<unsigned>(parts), static_cast<unsigned>(a.rows));
-    const int bins = fb_bins(a.vocab);
+    const int bins = a.fo_bins;
+    if (a.row_params) {
+        const dim3 all(static_cast<unsigned>(a.rows));
+        switch (bins / kFT) {
+            case 2: hipLaunchKernelGGL(fb_row_kernel<2>, all, dim3(kFT), 0, stream, a); break;
+            case 4: hipLaunchKernelGGL(fb_row_kernel<4>, all, dim3(kFT), 0, stream, a); break;
+            case 8: hipLaunchKernelGGL(fb_row_kernel<8>, all, dim3(kFT), 0, stream, a); break;
+            default: hipLaunchKernelGGL(fb_row_kernel<16>, all, dim3(kFT), 0, stream, a); break;
+        }
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(fb_range_kernel, grid, dim3(kFT), 0, stream, a);
     hipLaunchKernelGGL(fb_exps_kernel, grid, dim3(kFT), 0, stream, a);
     const dim3 rows(static_cast<unsigned>(a.rows));

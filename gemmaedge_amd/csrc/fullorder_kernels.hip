@@ -3144,11 +3144,9 @@ hipError_t sorted_pass(const DevArgs& a, hipStream_t stream) {
     int64_t per64 = std::min<int64_t>(a.fo_capacity / stride, a.rows);
     // f32 rows with k = V need no sort (fullorder_binned.hip); the sort-based
     // kernels then serve the rows it leaves. Shared parameters with
-    // 1024 < top_k < V go to them straight away, and calls with per-row
-    // parameters: the host cannot tell whether any row needs this path, and its
-    // launches cost 20 us when every row leaves at once.
-    const bool binned = std::is_same<T, float>::value && !a.fo_fallback && a.fo_tiles != nullptr && !a.row_params &&
-                        (a.params.top_k == 0u || a.params.top_k >= static_cast<uint32_t>(a.vocab)) &&
+    // 1024 < top_k < V go to them straight away.
+    const bool binned = std::is_same<T, float>::value && !a.fo_fallback && a.fo_tiles != nullptr &&
+                        (a.row_params || a.params.top_k == 0u || a.params.top_k >= static_cast<uint32_t>(a.vocab)) &&
                         a.fo_tiles_words >= fb_row_words(a.vocab);
     if (binned) {
         per64 = std::min(per64, a.fo_tiles_words / fb_row_words(a.vocab));

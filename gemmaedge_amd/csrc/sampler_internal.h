@@ -81,6 +81,7 @@ struct DevArgs {
     int64_t fo_capacity;          // items (and aux, pre entries) in the workspace
     uint32_t* fo_tiles;           // [fo_tiles_words] f32 rows' per-tile counts (many-workgroup sort) or bins (no sort)
     int64_t fo_tiles_words;
+    int32_t fo_bins;              // f32 rows without a sort: histogram bins per row
     // Full-order fallback pass (bf16 rows with more unique penalised ids than
     // fo_extras_cap): the sort-based kernels serve only the rows the first
     // pass flagged. fo_row0: the first call row of a slice of rows.
@@ -110,17 +111,25 @@ inline int64_t fo_items_stride_f32(int vocab) { return (static_cast<int64_t>(voc
 constexpr int fo_split_tiles(int vocab) { return (vocab + 4095) / 4096; }
 constexpr int64_t fo_tile_words(int tiles) { return static_cast<int64_t>(tiles) * (256 + 1 + 4); }
 
-// f32 rows without a sort (fullorder_binned.hip): histogram bins per row (about
-// one per 16 tokens), and the words of a row's area in fo_tiles.
+// f32 rows without a sort (fullorder_binned.hip): histogram bins per row, about
+// one per 16 tokens, at most 8,192 for few rows: there the plan, one workgroup
+// per row, is on the critical path (one row of V = 262,144: plan 36 -> 23 us,
+// order 6 -> 13; 64 rows 41 -> 26 and 19 -> 14), while many near-uniform rows
+// pay for the tokens of wider bins (256 rows: collect, order and draw 286 -> 363
+// us, plan 56 -> 37). And the words of a row's area in fo_tiles.
 constexpr int kFbMaxBins = 16384;
 constexpr int kFbParts = 64;    // workgroups that stream one row, at most
 constexpr int kFbSegs = 4096;   // expanded bins of one row, at most
 constexpr int kFbSegWords = 10; // words of one's record
-__host__ __device__ constexpr int fb_bins(int vocab) {
-    return vocab >= 131072 ? kFbMaxBins : vocab >= 65536 ? kFbMaxBins / 2 : vocab >= 32768 ? kFbMaxBins / 4 : kFbMaxBins / 8;
+constexpr int kFbManyRows = 128;
+constexpr int fb_bins(int vocab, int rows) {
+    return vocab >= 131072 && rows >= kFbManyRows ? kFbMaxBins
+           : vocab >= 65536                       ? kFbMaxBins / 2
+           : vocab >= 32768                       ? kFbMaxBins / 4
+                                                  : kFbMaxBins / 8;
 }
 __host__ __device__ constexpr int64_t fb_row_words(int vocab) {
-    return fb_bins(vocab) + 6 * kFbParts + 64 + kFbMaxBins / 32 + kFbSegWords * (kFbSegs + 2);
+    return (vocab >= 131072 ? kFbMaxBins : kFbMaxBins / 2) + 6 * kFbParts + 64 + kFbMaxBins / 32 + kFbSegWords * (kFbSegs + 2);
 }
 
 // The row's parameters: the shared ones, or its entry of row_params.
