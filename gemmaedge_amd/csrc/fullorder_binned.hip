@@ -61,7 +61,7 @@ constexpr uint32_t kLeast = 0x2f800000u;  // 2^-32: smaller exps share the last 
 constexpr uint32_t kFbHead = 1024;     // tokens always expanded
 constexpr int kFbWaveSeg = 512;        // tokens of a bin that one wave orders
 constexpr uint32_t kFbSegMost = 4096;  // tokens of an expanded bin at most
-constexpr double kFbDrift = 0x1p-13;   // the plan's relative margin on a float sum
+constexpr double kFbDrift = 0x1p-14;   // the plan's relative margin on a float sum
 
 // One expanded bin. What the chains add (cumulative) or take off (walk) for the
 // bins between two replayed ones is a sum of whole ulps of one binade.
@@ -108,10 +108,9 @@ __device__ __forceinline__ FbRow fb_row(const DevArgs& a, int row, int bins) {
     r.seg = reinterpret_cast<FbSeg*>(r.mask + kFbMaxBins / 32);
     return r;
 }
-// The row's exps, in the upper half of its items (fb_half() items are left).
-__device__ __forceinline__ int64_t fb_half(const DevArgs& a) { return a.fo_items_stride / 2; }
+// The row's exps.
 __device__ __forceinline__ float* fb_exp_array(const DevArgs& a, int row) {
-    return reinterpret_cast<float*>(a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride + fb_half(a));
+    return a.fo_aux + static_cast<int64_t>(row) * a.fo_items_stride;
 }
 __device__ __forceinline__ uint32_t fb_bin(float pe, uint32_t shift, uint32_t bins) {
     return min((kOne - f2u(pe)) >> shift, bins - 1u);
@@ -504,9 +503,16 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
     auto hi_pe = [&](int b) { return u2f(kOne - (static_cast<uint32_t>(b) << shift)); };
     auto lo_pe = [&](int b) { return b == kBins - 1 ? 0.0f : u2f(kOne - (static_cast<uint32_t>(b + 1) << shift) + 1u); };
     auto mid = [&](int b) { return 0.5f * (lo_pe(b) * inv + hi_pe(b) * inv); };
-    auto rounded = [&](int b, float c, double acc) {  // bin b's addends in the binade of acc
-        const int e = max(fb_expo(acc), 64);          // (below 2^-63 nothing rounds)
-        return c * __builtin_ldexpf(__builtin_rintf(__builtin_ldexpf(mid(b), 150 - e)), e - 150);
+    // Bin b's addends in the binade of acc: their mean number of ulps, taken as
+    // evenly spread over the bin (rounding its middle instead drifts by 1e-4 over
+    // the bins whose addends differ by about half an ulp).
+    auto rounded = [&](int b, float c, double acc) {
+        const int e = max(fb_expo(acc), 64);  // (below 2^-63 nothing rounds)
+        const float yl = __builtin_ldexpf(lo_pe(b) * inv, 150 - e), yh = __builtin_ldexpf(hi_pe(b) * inv, 150 - e);
+        const float nl = __builtin_rintf(yl), nh = __builtin_rintf(yh), span = yh - yl;
+        float y = nl;
+        if (nl != nh) y = span > 1.0f || yh > 4096.0f ? 0.5f * (yl + yh) : nl + (yh - (nh - 0.5f)) / span * (nh - nl);
+        return c * __builtin_ldexpf(y, e - 150);
     };
     // f(bin, its padded index, its count) for this thread's bins that hold any.
     auto each = [&](auto&& f) {
@@ -590,7 +596,10 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
         mass_hi = max(mass_hi, 2.0 * q_first);
     }
     const double u = static_cast<double>(a.uniforms[row]);
-    const double c_lo = u * mass_lo * (1.0 - 2.0 * kFbDrift), c_hi = u * mass_hi * (1.0 + 2.0 * kFbDrift);
+    // (a sum that top_p stops is the float itself: only one that ends at the cut
+    // or the row's end has drifted)
+    const double c_lo = u * mass_lo * (1.0 - (mass_lo < tp ? kFbDrift : 0x1p-20));
+    const double c_hi = u * mass_hi * (1.0 + (mass_hi < tp ? kFbDrift : 0x1p-20));
     const double c_mid = 0.5 * (c_lo + c_hi);
     // What the walk has taken off before each bin.
     // (threads whose bins no chain reaches have nothing more to find)
@@ -625,7 +634,8 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
             bool ex = rc || !fb_alike(ql, qh, ea, dc);
             int ew = 0;
             bool rw = false;
-            const double w_hi = c_hi * (1.0 + kFbDrift) - W, w_lo = c_lo - c_hi * kFbDrift - W1;
+            const double slack = c_hi * kFbDrift + (head ? __builtin_fabs(corr) : 0.0);
+            const double w_hi = c_hi + slack - W, w_lo = c_lo - slack - W1;
             if (w_hi > 0.0) {
                 ew = fb_expo(w_hi);
                 const bool draw = !(w_lo > 0.0);  // the walk may stop here
@@ -661,7 +671,7 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
     uint32_t off = n_items, seg = n_seg, elems_at = n_elem, unused = 0, none_all;
     fb_scan_3<kFW>(off, seg, cum, sh.sd, sh.su, sh.sv, G, segs, cum_all);
     fb_scan_3<kFW>(elems_at, unused, walk, sh.sd, sh.su, sh.sv, elems, none_all, walk_all);
-    if (sh.bad || static_cast<int64_t>(G) + 1 > fb_half(a) || segs > static_cast<uint32_t>(kFbSegs)) {
+    if (sh.bad || segs > static_cast<uint32_t>(kFbSegs)) {
         if (tid == 0) meta[kMetaStatus] = kStatusToSort;
         return;
     }
@@ -926,7 +936,7 @@ __device__ __forceinline__ void fb_order(const DevArgs& a, int row, int block, i
 //    added at once. One wave takes the lists 64 elements a step. Then the
 //    near-boundary flag and the token. Latency-bound: about 150 steps of
 //    dependent work per chain for near-uniform rows.
-constexpr int kDrawList = 8192;     // replayed elements of one chain
+constexpr int kDrawList = 14336;    // replayed elements of one chain
 constexpr int kDrawRegions = 512;   // their regions
 constexpr int kDrawTies = 4096;     // tokens of one exp (kFbSegMost)
 
@@ -942,7 +952,7 @@ struct DrawList {
     uint32_t expo[kDrawRegions + 1];   // the accumulator's binade before it
     int n;                             // regions
 };
-static_assert(kDrawList * 4 == kDrawTies * 8, "the union");
+static_assert(kDrawList * 4 >= kDrawTies * 8, "the union");
 struct DrawShared {
     DrawList list[2];  // cumulative, walk
     double sd[32];
