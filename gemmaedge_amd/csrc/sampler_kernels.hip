@@ -2843,7 +2843,8 @@ constexpr uint32_t kPlPer = 6;          // entry words per merging thread per li
 constexpr uint32_t kPlMaxEntries = 62;  // entry positions of one list at most
 constexpr uint64_t kPlFiller = 1;    // an unused entry position (value key 0: never a candidate)
 constexpr uint64_t kPlOverflow = ~uint64_t{0}; // header of a list that could not hold its candidates
-constexpr uint32_t kPlCand = 4;         // candidates a lane stages (more: the list overflows)
+constexpr uint32_t kPlCand = 4;         // candidates a lane lists (more: the wave raises its bound)
+constexpr uint32_t kPlStage = 6;        // candidates a lane stages (more: the list overflows)
 constexpr uint32_t kPlSpins = 1u << 22; // about 4 s of polling; every awaited workgroup has started
 
 // Entry positions per list for a row of nl = 4 * cpr lists (nl <= 64). An
@@ -2862,7 +2863,10 @@ __device__ __forceinline__ uint32_t pl_entries(uint32_t nl) {
 // Deterministic, so every workgroup of a row agrees.
 __device__ __forceinline__ uint32_t pl_rank(uint32_t k, int cpr, uint32_t entries) {
     const float mu = spec_mu(k, cpr);
-    const uint32_t q = static_cast<uint32_t>(ceilf((mu + 2.0f * __builtin_amdgcn_sqrtf(mu) + 4.0f) * 0.25f));
+    // (few chunks: each holds a larger share of the top k, and 2 sqrt(mu) left
+    // 1 row in 30 short at 2 chunks, k = 64; 2.5 leaves 1 in 500)
+    const float dev = cpr <= 4 ? 2.5f : 2.0f;
+    const uint32_t q = static_cast<uint32_t>(ceilf((mu + dev * __builtin_amdgcn_sqrtf(mu) + 4.0f) * 0.25f));
     return min(max(q, 1u), max(min(16u, entries / 2u), 1u));
 }
 
@@ -3015,9 +3019,9 @@ __global__ __launch_bounds__(kBlock, 4) void stream_kernel(DevArgs a) {
     // A wave without a bound of its own lists every element above -inf.
     const float floor_v = tlo ? key_value(tau_lo) : -FLT_MAX;
     uint64_t* seg = sh.stage + wave * kSeg;
-    uint64_t* cmp = seg + kPlCand * 64;            // compacted candidates (at most kPlMaxEntries)
+    uint64_t* cmp = seg + kPlStage * 64;           // compacted candidates (at most kPlMaxEntries)
     constexpr uint32_t kDummy = kSeg - 64;          // per-lane dummy words
-    static_assert(kPlCand * 64 + kPlMaxEntries <= kDummy, "staging layout");
+    static_assert(kPlStage * 64 + kPlMaxEntries <= kDummy, "staging layout");
     const uint32_t ebase = static_cast<uint32_t>(c0 + tid * W);
     uint32_t cnt = 0;
 #pragma unroll
@@ -3029,8 +3033,8 @@ __global__ __launch_bounds__(kBlock, 4) void stream_kernel(DevArgs a) {
             const float x = value(s);
             const bool c = x >= floor_v;
             const uint32_t e = ebase + static_cast<uint32_t>((s / W) * kBlock * W + s % W);
-            const uint32_t slot = (c && cnt < kPlCand) ? 64u * cnt + static_cast<uint32_t>(lane)
-                                                       : kDummy + static_cast<uint32_t>(lane);
+            const uint32_t slot = (c && cnt < kPlStage) ? 64u * cnt + static_cast<uint32_t>(lane)
+                                                        : kDummy + static_cast<uint32_t>(lane);
             seg[slot] = (static_cast<uint64_t>(f2u(x)) << 32) | e;
             cnt += c ? 1u : 0u;
         }
@@ -3038,9 +3042,10 @@ __global__ __launch_bounds__(kBlock, 4) void stream_kernel(DevArgs a) {
     const uint64_t m0 = __ballot(cnt > 0u), m1 = __ballot(cnt > 1u), m2 = __ballot(cnt > 2u), m3 = __ballot(cnt > 3u);
     const uint32_t p0 = static_cast<uint32_t>(__popcll(m0)), p1 = static_cast<uint32_t>(__popcll(m1));
     const uint32_t p2 = static_cast<uint32_t>(__popcll(m2)), p3 = static_cast<uint32_t>(__popcll(m3));
-    const uint32_t n_w = p0 + p1 + p2 + p3;
-    const bool overflow = __ballot(cnt > kPlCand) != 0ull || n_w > ne;
-    if (!overflow) {
+    uint32_t n_w = p0 + p1 + p2 + p3;
+    uint32_t thr = tau_lo;  // the bound this wave lists down to
+    bool overflow = __ballot(cnt > kPlCand) != 0ull || n_w > ne;
+    if (__builtin_expect(!overflow, 1)) {
         uint64_t y0 = 0, y1 = 0, y2 = 0, y3 = 0;
         if (cnt > 0u) y0 = seg[lane];
         if (cnt > 1u) y1 = seg[64 + lane];
@@ -3050,6 +3055,34 @@ __global__ __launch_bounds__(kBlock, 4) void stream_kernel(DevArgs a) {
         if (cnt > 1u) cmp[p0 + lanes_below(m1)] = y1;
         if (cnt > 2u) cmp[p0 + p1 + lanes_below(m2)] = y2;
         if (cnt > 3u) cmp[p0 + p1 + p2 + lanes_below(m3)] = y3;
+    } else if (tlo != 0u && __ballot(cnt > kPlStage) == 0ull) {
+        // Too many for the list (one wave's bound far below the others', or a
+        // lane with many of them: one row in 200 to 400 at V = 262,144, k = 40
+        // to 64), but all staged: list them down to the wave's own q-th lane
+        // maximum instead, else to its largest. The header says so, the row's
+        // bound rises a little, and the row still merges; before, the row
+        // went to the rescans (one such row made a 64-row call 105 us, not 20).
+        uint32_t big = 0u;
+#pragma unroll 1
+        for (uint32_t c = 0; c < cnt; ++c)
+            big = max(big, order_key(u2f(static_cast<uint32_t>(seg[64u * c + static_cast<uint32_t>(lane)] >> 32))));
+        big = wave::max_u32(big);
+#pragma unroll 1
+        for (int t = 0; t < 2 && overflow; ++t) {
+            thr = t == 0 ? tlo : big;
+            const float fl = key_value(thr);
+            n_w = 0u;
+#pragma unroll 1
+            for (uint32_t c = 0; c < kPlStage; ++c) {
+                const uint64_t y = c < cnt ? seg[64u * c + static_cast<uint32_t>(lane)] : 0ull;
+                const bool in = c < cnt && u2f(static_cast<uint32_t>(y >> 32)) >= fl;
+                const uint64_t m = __ballot(in);
+                const uint32_t at = n_w + lanes_below(m);
+                if (in && at < ne) cmp[at] = y;
+                n_w += static_cast<uint32_t>(__popcll(m));
+            }
+            overflow = n_w > ne;
+        }
     }
     wave_lds_sync();
     // 5. Final keys (one softcap round for the wave: lane i < n_w takes
@@ -3070,7 +3103,7 @@ __global__ __launch_bounds__(kBlock, 4) void stream_kernel(DevArgs a) {
             pen = ((s_pbits[off >> 5] >> (off & 31)) & 1u) != 0u;
         }
     } else if (lane == 63) {
-        xv = tau_lo != 0xffffffffu ? key_value(tau_lo) : -INFINITY;
+        xv = tau_lo != 0xffffffffu ? key_value(thr) : -INFINITY;
     }
     float f = softcap(xv, rc.cap);
     if (pen) f = penalize(f, rc.r);
