@@ -34,13 +34,14 @@
 // kFbSegMost tokens).
 //
 // Measured against the radix sort it replaces (whole calls, V = 262,144): one
-// row 245 -> 106 us, 64 rows 824 -> 216 us, 512 near-uniform rows 4,822 ->
-// 1,281 us; of the last, per 256 rows: range 63, exps 237, plan 55, collect 92,
-// order 105, draw 87 us.
+// row 241 -> 97 us, 64 rows 822 -> 185 us, 512 near-uniform rows 4,820 ->
+// 1,063 us; of the last, per 256 rows: range 64, exps 171, plan 57, collect 92,
+// order 66, draw 81 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "chain_math.h"
 #include "fullorder_common.h"
@@ -786,11 +787,37 @@ __device__ __forceinline__ void fb_collect(const DevArgs& a, int row, int part, 
     }
 }
 
+// Each key's rank among a wave's n keys (kV per lane, key v of lane l the
+// (64 v + l)-th; zero past n): how many are larger.
+template <int kV>
+__device__ __forceinline__ void fb_rank(const uint32_t (&key)[kV], uint32_t n, uint32_t (&rank)[kV]) {
+#pragma unroll
+    for (int v = 0; v < kV; ++v) rank[v] = 0;
+#pragma unroll
+    for (int w = 0; w < kV; ++w) {
+        const int m = min(static_cast<int>(n) - 64 * w, 64);
+#pragma unroll 1
+        for (int c = 0; c < m; c += 8) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t k = wave::readlane(key[w], c + i);
+#pragma unroll
+                for (int v = 0; v < kV; ++v) rank[v] += k > key[v] ? 1u : 0u;
+            }
+        }
+    }
+}
+
 // 5. Each expanded bin: the ulps its tokens add where it is not replayed (a
 //    bin with a tie among them is replayed after all), and a replayed bin's
 //    tokens by (exp descending, index ascending): one wave per bin by counting
-//    the larger keys (every lane's up to eight keys against an LDS broadcast),
-//    the workgroup by a bitonic sort for the rare larger ones.
+//    the larger keys, the workgroup by a bitonic sort for the rare larger ones.
+//    Bound by the counting. Exps of one bin differ in `shift` low bits only:
+//    where these and the token's index fit 32 bits (near-uniform rows, whose
+//    bins hold up to 120 tokens) the keys are ranked as 32-bit words from
+//    registers; other bins rank 64-bit keys against an LDS broadcast.
+//    256 near-uniform rows of V = 262,144: 98 us with 64-bit keys for all, 66 so;
+//    16 workgroups a row measure the same, 5 (all resident at once) 79.
 struct OrderShared {
     uint64_t stage[kFbSegMost];
 };
@@ -806,6 +833,9 @@ __device__ __forceinline__ void fb_order(const DevArgs& a, int row, int block, i
     const FbRow r = fb_row(a, row, a.fo_bins);
     const int segs = static_cast<int>(r.scal[kScSegs]);
     const float inv = u2f(r.scal[kScInv]);
+    const uint32_t shift = r.scal[kScShift], last_bin = static_cast<uint32_t>(a.fo_bins) - 1u;
+    const int idx_bits = 32 - __clz(a.vocab - 1);
+    const bool narrow = static_cast<int>(shift) + idx_bits <= 32;
     uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
     uint64_t* mine = sh.stage + wave * kWaveSeg;
     bool large = false;
@@ -867,7 +897,36 @@ __device__ __forceinline__ void fb_order(const DevArgs& a, int row, int block, i
             }
         }
         if (!(info & (kSegReplayCum | kSegReplayWalk))) continue;
-        if (n <= 64u) {
+        // (the last bin holds every smaller exp too)
+        const bool words = narrow && n <= 256u &&
+                           wave::readlane(fb_bin(u2f(static_cast<uint32_t>(key0 >> 32)), shift, last_bin + 1u), 0) != last_bin;
+        auto by_words = [&](auto kv) {
+            constexpr int kV = decltype(kv)::value;
+            uint64_t key[kV];
+            uint32_t word[kV], rank[kV];
+#pragma unroll
+            for (int v = 0; v < kV; ++v) {
+                const uint32_t i = static_cast<uint32_t>(v) * 64u + static_cast<uint32_t>(lane);
+                key[v] = v == 0 ? key0 : items[off + min(i, n - 1u)];
+            }
+            // ((2^shift - 1 - the exp's distance into the bin), then the index's complement)
+            const uint32_t below = (1u << shift) - 1u, idx_mask = (1u << idx_bits) - 1u;
+#pragma unroll
+            for (int v = 0; v < kV; ++v) {
+                const uint32_t hi = below - ((kOne - static_cast<uint32_t>(key[v] >> 32)) & below);
+                const bool in = static_cast<uint32_t>(v) * 64u + static_cast<uint32_t>(lane) < n;
+                word[v] = in ? (hi << idx_bits) | (static_cast<uint32_t>(key[v]) & idx_mask) : 0u;
+            }
+            fb_rank<kV>(word, n, rank);
+#pragma unroll
+            for (int v = 0; v < kV; ++v)
+                if (static_cast<uint32_t>(v) * 64u + static_cast<uint32_t>(lane) < n) items[off + rank[v]] = key[v];
+        };
+        if (words) {
+            if (n <= 64u) by_words(std::integral_constant<int, 1>{});
+            else if (n <= 128u) by_words(std::integral_constant<int, 2>{});
+            else by_words(std::integral_constant<int, 4>{});
+        } else if (n <= 64u) {
             uint32_t rank = 0;
             for (uint32_t j = 0; j < n; ++j) rank += wave::readlane64(key0, static_cast<int>(j)) > key0 ? 1u : 0u;
             if (static_cast<uint32_t>(lane) < n) items[off + rank] = key0;

@@ -75,6 +75,24 @@ def test_ends_and_cuts(sampler, kind, params):
     _check(sampler, w)
 
 
+@pytest.mark.parametrize("vocab,top", [(W.VOCAB, 0.0), (131071, 0.0), (65537, 0.0), (W.VOCAB, 1.5), (W.VOCAB, 12.0)])
+def test_bins_of_every_size(sampler, vocab, top):
+    # Near-uniform rows whose bins hold from one token to a few hundred, the
+    # chains' binade changes and the draw at many places among them; with `top`
+    # a few larger values widen the bins until a key takes more than 32 bits.
+    # Quantised rows: equal exps, told apart by the index.
+    rng = np.random.default_rng(vocab + int(top))
+    u = np.linspace(0.01, 0.99, 9).astype(np.float32)
+    for sigma, step in ((0.1, 0.0), (0.02, 0.0), (0.3, 0.0), (0.1, 2.0**-16)):
+        x = (rng.standard_normal((9, vocab)) * sigma).astype(np.float32)
+        if step:
+            x = (np.round(x / step) * step).astype(np.float32)
+        x[:, :3] += np.float32(top)
+        for top_p in (0.6, 0.95):
+            _check(sampler, small_workload(f"bins-{sigma}-{step}-{top_p}", x,
+                                           dict(temperature=1.1, top_k=0, top_p=top_p, softcap=30.0), uniforms=u))
+
+
 def test_ties_and_quantised_values(sampler):
     # bf16 values in f32 (hundreds of equal tokens a value), and a coarser grid
     rng = np.random.default_rng(3)
