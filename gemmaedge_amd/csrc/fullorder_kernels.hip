@@ -601,7 +601,9 @@ __global__ __launch_bounds__(kThreads) void fo_hist_kernel(DevArgs a) {
 
 // ---- kernel 1, f32 rows: every token's final key, sorted --------------------
 //
-// An f32 row can hold V distinct values, so its items come from a sort of
+// Rows with 1024 < k < V, and rows that the sort-free path
+// (fullorder_binned.hip, k = V) leaves. An f32 row can hold V
+// distinct values, so its items come from a sort of
 // the final keys of all its tokens (softcap, then the penalty on marked ids),
 // complemented so that ascending order is the reference's descending one.
 // One 1024-thread workgroup per row runs a stable LSD radix sort, 8 bits per
@@ -963,7 +965,8 @@ __global__ __launch_bounds__(kThreads) void fo_sort_kernel(DevArgs a) {
 // ---- f32 rows over many workgroups: the same items, tile by tile -----------
 //
 // The sort above gives each row one workgroup; with few rows most of the GPU
-// idles while its passes run. Here a row's keys are cut into tiles of
+// idles while its passes run (shared parameters with 1024 < k < V come here).
+// Here a row's keys are cut into tiles of
 // kSTile keys, one 256-thread workgroup per (tile, row), and each step of the
 // sort is a kernel of its own: the kernel boundaries order every exchange
 // between workgroups, so no workgroup waits for another. The results are
