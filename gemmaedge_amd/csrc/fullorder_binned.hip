@@ -1282,16 +1282,20 @@ __device__ __forceinline__ void fb_draw(const DevArgs& a, int row, int parts, Dr
         double before = 0.0;
         bool nb = false, na = false;
         if (pos > 0u) {
-            if (item < draw0 || item >= draw1) {
+            // (item == pos: every token before it is in the list, whatever the
+            // plan expected: a draw one token before its range sent 3 peaked rows in
+            // 15,000 to the sort)
+            const bool head = static_cast<uint32_t>(item) == pos;
+            if (!head && (item < draw0 || item >= draw1)) {
                 ok = false;
             } else {
                 double t = 0.0;
-                for (int i = draw0 + tid; i < item; i += kThreads)
+                for (int i = (head ? 0 : draw0) + tid; i < item; i += kThreads)
                     t += static_cast<double>(u2f(static_cast<uint32_t>(items[i] >> 32)) * inv);
                 t = wave::sum_f64(t);
                 if (lane == 0) sh.sd[wave] = t;
                 __syncthreads();
-                before = wave::sum_f64(lane < parts ? r.pbef[lane] : 0.0);
+                before = head ? 0.0 : wave::sum_f64(lane < parts ? r.pbef[lane] : 0.0);
                 for (int v = 0; v < kWaves; ++v) before += sh.sd[v];
                 ok = near_decided(ch, before, near_sum_error(pos), nb);
             }
