@@ -94,7 +94,8 @@ struct FbRow {
     uint32_t* mask;   // [bins / 32] expanded bins
     FbSeg* seg;       // [kFbSegs + 1] the expanded bins, in order, and the list's end
 };
-enum : int { kScShift = 0, kScInv, kScDrawBin, kScDrawItem, kScDrawEnd, kScSegs, kScCut, kScalWords = 64 };
+// (kScLarge: fb_order met a bin too large to order, so the draw leaves the row)
+enum : int { kScShift = 0, kScInv, kScDrawBin, kScDrawItem, kScDrawEnd, kScSegs, kScCut, kScLarge, kScalWords = 64 };
 
 __device__ __forceinline__ FbRow fb_row(const DevArgs& a, int row, int bins) {
     uint32_t* w = a.fo_tiles + static_cast<int64_t>(row) * fb_row_words(a.vocab);
@@ -709,6 +710,7 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
         r.scal[kScDrawItem] = sh.off0;
         r.scal[kScDrawEnd] = none ? 0u : sh.off1;
         r.scal[kScSegs] = segs;
+        r.scal[kScLarge] = 0u;
         // whether the list ends where the reference's sums do: the row's end,
         // or the bin of the min-p cut
         r.scal[kScCut] = elems == static_cast<uint32_t>(V) || (cut != 0xffffffffu && sh.cut_lo * (1.0 - kFbDrift) < tp) ? 1u : 0u;
@@ -828,8 +830,7 @@ __device__ __forceinline__ void fb_order(const DevArgs& a, int row, int block, i
     constexpr uint32_t kWaveSeg = kMy * 64;
     const int tid = threadIdx.x, lane = __lane_id(), wave = tid >> 6;
     ge_sample_params p;
-    uint32_t* meta = fb_meta(a, row);
-    if (!fb_serves(a, row, p) || meta[kMetaStatus] != kStatusOk) return;
+    if (!fb_serves(a, row, p) || fb_meta(a, row)[kMetaStatus] != kStatusOk) return;
     const FbRow r = fb_row(a, row, a.fo_bins);
     const int segs = static_cast<int>(r.scal[kScSegs]);
     const float inv = u2f(r.scal[kScInv]);
@@ -953,7 +954,9 @@ __device__ __forceinline__ void fb_order(const DevArgs& a, int row, int block, i
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         } else {
             large = true;
-            if (n > kFbSegMost && lane == 0) meta[kMetaStatus] = kStatusToSort;
+            // (not the status word: other waves and workgroups of this kernel still
+            // read that, and must all go on to the barriers below)
+            if (n > kFbSegMost && lane == 0) r.scal[kScLarge] = 1u;
         }
       }
     }
@@ -1210,7 +1213,7 @@ __device__ __forceinline__ void fb_draw(const DevArgs& a, int row, int parts, Dr
     const float inv = u2f(r.scal[kScInv]);
     const int draw0 = static_cast<int>(r.scal[kScDrawItem]), draw1 = static_cast<int>(r.scal[kScDrawEnd]);
     const bool whole = r.scal[kScCut] != 0u;
-    bool ok = draw_lists<kThreads>(r, segs, items, inv, sh);
+    bool ok = r.scal[kScLarge] == 0u && draw_lists<kThreads>(r, segs, items, inv, sh);
     const float u = a.uniforms[row];
     float choice = 0.0f;
     if (ok && wave == 0) {

@@ -17,6 +17,7 @@
 #include <string>
 
 #include "../../include/gemmaedge_sampler.h"
+#include "fullorder_common.h"
 #include "sampler_internal.h"
 #include "sampler_validate.h"
 
@@ -402,6 +403,24 @@ int ge_sample_noalloc(void* stream, const ge_sample_args* args) {
     ws.tickets = static_cast<uint32_t*>(p);
     ws.slots = reinterpret_cast<uint64_t*>(static_cast<char*>(p) + kTicketBytes);
     return sample_on(ws, stream, *args);
+}
+
+// For tests (not declared in the public header): which of the last f32 call's
+// full-order rows [0, rows) were left to the sort by the sort-free path (1) or
+// served by it (0). Calls of more rows than one slice of the workspace report
+// their last slice. Waits for the device.
+int ge_test_rows_left(ge_sampler* s, int rows, int32_t* left) {
+    if (!s || !left || rows < 1 || rows > s->max_rows || !s->fo_meta)
+        return fail(GE_ERR_INVALID_ARG, "sampler, left or rows");
+    DeviceGuard guard(s->device);
+    if (!guard.ok) return fail(GE_ERR_DEVICE, "hipSetDevice(%d) failed", s->device);
+    hipError_t e = hipDeviceSynchronize();
+    if (e == hipSuccess)
+        e = hipMemcpy2D(left, sizeof(int32_t), s->fo_meta + ge::kMetaStatus, ge::kMetaWords * sizeof(uint32_t),
+                        sizeof(uint32_t), static_cast<size_t>(rows), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return hip_fail(e, "ge_test_rows_left");
+    for (int r = 0; r < rows; ++r) left[r] = left[r] == static_cast<int32_t>(ge::kStatusFallback) ? 1 : 0;
+    return GE_OK;
 }
 
 }  // extern "C"

@@ -28,6 +28,19 @@ def run_gpu(sampler, w: W.Workload):
     return tokens.cpu().numpy(), probs.cpu().numpy(), flags.cpu().numpy()
 
 
+def rows_left(sampler, rows: int):
+    """Which of the last f32 call's full-order rows the sort-free path left to the sort."""
+    import ctypes
+
+    from gemmaedge_amd import load_library
+    from gemmaedge_amd.sampler import GE_OK, last_error
+
+    left = (ctypes.c_int32 * rows)()
+    rc = load_library().ge_test_rows_left(sampler._h, rows, left)
+    assert rc == GE_OK, last_error()
+    return [r for r in range(rows) if left[r]]
+
+
 def run_oracle(w: W.Workload, nthreads: int = 0):
     hist = w.history if w.history.size else None
     offs = w.offsets if w.history.size else None
