@@ -1011,7 +1011,7 @@ struct DrawList {
     uint32_t pos[kDrawRegions + 1];    // its first list position; [n]: the list's length
     uint32_t item[kDrawRegions + 1];
     uint32_t elem[kDrawRegions + 1];
-    uint32_t expo[kDrawRegions + 1];   // the accumulator's binade before it
+    uint32_t expo[kDrawRegions + 1];   // the accumulator's binade before it (0: no bins lie between, or none that add)
     int n;                             // regions
 };
 static_assert(kDrawList * 4 >= kDrawTies * 8, "the union");
@@ -1036,7 +1036,7 @@ __device__ __forceinline__ bool draw_lists(const FbRow& r, int segs, const uint6
     const int count = segs + 1;  // with the list's end
     const int per = (count + kThreads - 1) / kThreads;
     const int s0 = min(tid * per, count), s1 = min(s0 + per, count);
-    // f(record, chain, replayed, begins a region)
+    // f(record, chain, replayed, begins a region, follows the replayed tokens before it)
     auto each = [&](auto&& f) {
         const FbSeg p = r.seg[max(s0 - 1, 0)];
         bool prev[2];
@@ -1053,7 +1053,8 @@ __device__ __forceinline__ bool draw_lists(const FbRow& r, int segs, const uint6
 #pragma unroll
                 for (int x = 0; x < 2; ++x) {
                     const bool rep = (g[v].info & kReplay[x]) != 0u;
-                    f(g[v], x, rep, rep && !(prev[x] && next == g[v].elem && g[v].n != 0u));
+                    const bool follows = prev[x] && next == g[v].elem;  // no bins between
+                    f(g[v], x, rep, rep && !(follows && g[v].n != 0u), follows);
                     prev[x] = rep;
                 }
                 next = g[v].elem + g[v].n;
@@ -1062,7 +1063,7 @@ __device__ __forceinline__ bool draw_lists(const FbRow& r, int segs, const uint6
     };
     double t[2] = {0.0, 0.0};  // the ulps of the expanded bins that are not replayed
     uint32_t n[2] = {0, 0}, at[2] = {0, 0};
-    each([&](const FbSeg& g, int x, bool rep, bool start) {
+    each([&](const FbSeg& g, int x, bool rep, bool start, bool) {
         if (rep) n[x] += g.n;
         else t[x] += static_cast<double>(x ? g.swalk : g.scum);
         at[x] += start ? 1u : 0u;
@@ -1098,14 +1099,14 @@ __device__ __forceinline__ bool draw_lists(const FbRow& r, int segs, const uint6
     }
     if (max(n_all[0], n_all[1]) > static_cast<uint32_t>(kDrawList) || max(r_all[0], r_all[1]) > static_cast<uint32_t>(kDrawRegions))
         return false;
-    each([&](const FbSeg& g, int x, bool rep, bool start) {
+    each([&](const FbSeg& g, int x, bool rep, bool start, bool follows) {
         DrawList& l = sh.list[x];
         if (start) {
             l.before[at[x]] = t[x] + (x ? g.walk : g.cum);
             l.pos[at[x]] = n[x];
             l.item[at[x]] = g.item;
             l.elem[at[x]] = g.elem;
-            l.expo[at[x]] = x ? (g.info >> 8) & 0xffu : g.info & 0xffu;
+            l.expo[at[x]] = follows ? 0u : x ? (g.info >> 8) & 0xffu : g.info & 0xffu;
             ++at[x];
         }
         if (rep) n[x] += g.n;
@@ -1147,10 +1148,15 @@ __device__ __forceinline__ int draw_chain(const DrawList& l, uint32_t& k, uint32
         const uint32_t tm = kDesc ? 0u : chain::threshold_bits(f2u(thr), b.uexp);
         if (k == rend) {  // the bins between this region and the next
             if (region + 1 >= l.n) return -1;
+            // The plan took them in one binade. In a higher one their ulps are
+            // others, unless they add nothing: then they add nothing there
+            // either. In a lower one they may add even where the plan's add
+            // nothing.
             const double jump = l.before[region + 1] - l.before[region];
-            if (jump != 0.0) {
+            const uint32_t planned = l.expo[region + 1], have = static_cast<uint32_t>(b.uexp + 150);
+            if (planned != 0u) {
                 const double m = static_cast<double>(b.m);
-                if (l.expo[region + 1] != static_cast<uint32_t>(b.uexp + 150)) return -1;
+                if (have < planned || (have > planned && jump != 0.0)) return -1;
                 if (kDesc ? m - jump < static_cast<double>(b.lo)
                           : (m + jump > static_cast<double>(chain::kHiF) || m + jump >= static_cast<double>(tm)))
                     return -1;

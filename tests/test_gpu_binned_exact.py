@@ -74,6 +74,28 @@ def sampler():
     s.close()
 
 
+def test_bins_that_add_nothing_in_the_expected_binade(sampler):
+    # Thousands of tokens a little below (k + 1/2) ulps: the sum falls 2e-3 short
+    # of 1.0, where an even spread of the addends would take it past 1.0. There
+    # the tail's addends (just above half an ulp of [1/2, 1)) would add nothing;
+    # in truth each adds an ulp.
+    inv = np.float32(4e-4)
+    k = np.array([89, 84, 80, 76, 72, 67, 63, 59, 46, 44, 42, 40, 31, 29, 27, 25, 24, 9, 8])
+    mid = _logits_below(inv, (k + 0.5) * U * (1 - 2e-6))
+    tail = np.log(np.linspace(5.6e-8, 4.4e-8, 24600) / float(inv)).astype(np.float32)
+    head = np.log(np.linspace(1.0, 0.1, 3480)).astype(np.float32)
+    head[0] = 0.0
+    values = np.concatenate([head, mid, tail])
+    counts = np.concatenate([np.ones(3480, int), np.full(18, 4222), [4000], np.ones(24600, int)])
+    row = _scaled_to(inv, values, counts, np.float32(-0.9))
+    rng = np.random.default_rng(1)
+    rng.shuffle(row)
+    u = np.array([0.001, 0.05, 0.1, 0.2, 0.3, 0.35, 0.5, 0.9], np.float32)
+    w = small_workload("gap", np.repeat(row[None], 8, 0), dict(temperature=1.0, top_k=0, top_p=2.0), uniforms=u)
+    print(f"[binned exact] {w.name} V={w.vocab}", flush=True)
+    assert_parity(w, run_gpu(sampler, w), run_oracle(w))
+
+
 def test_a_large_bin_of_ties(sampler):
     # 6,000 tokens of one value half way between two ulps of the sum: a bin that
     # the cumulative sum was to pass as whole ulps, and too large to order.
