@@ -467,7 +467,7 @@ struct PlanShared {
     double sd[kFW];
     uint32_t su[kFW], sv[kFW];
     uint32_t mask[kFbMaxBins / 32];
-    uint32_t bad, cut, stop, first, last, off0, off1;
+    uint32_t bad, cut, cut_elem, stop, first, last, off0, off1;
     double cut_lo, cut_hi;
     float stop_q;
 };
@@ -489,7 +489,7 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
     const double S = wave::sum_f64(lane < parts ? r.psum[lane] : 0.0);
     if (tid == 0) {
         sh.bad = 0u;
-        sh.cut = sh.stop = sh.first = 0xffffffffu;
+        sh.cut = sh.cut_elem = sh.stop = sh.first = 0xffffffffu;
         sh.last = 0u;
         sh.cut_lo = sh.cut_hi = 0.0;
         sh.stop_q = 0.0f;
@@ -619,6 +619,7 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
     uint32_t at = before;
     uint32_t seen = 0;  // how many of this thread's bins with tokens are (a prefix of them)
     uint32_t expo_end = 0;
+    const int e_first = fb_expo(q_first);
     // The walk's ulps per addend of an unexpanded bin.
     auto walk_ulps = [&](int b, int ew) -> uint32_t {
         return ew ? static_cast<uint32_t>(__builtin_floorf(__builtin_ldexpf(hi_pe(b) * inv, 150 - ew) + 0.5f)) : 0u;
@@ -627,16 +628,26 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
         const double W1 = W + static_cast<double>(rounded(b, static_cast<float>(c), c_mid - 0.5 * (A + A1)));
         const bool head = at < kFbHead;
         const double a_lo = A * (1.0 - kFbDrift), a_hi = A1 * (1.0 + kFbDrift);
-        if (head || (a_lo < tp && static_cast<uint32_t>(b) <= cut)) {
-            const float qh = hi_pe(b) * inv, ql = lo_pe(b) * inv;
-            const bool edge = head || static_cast<uint32_t>(b) == cut || a_hi >= tp;
-            const int ea = fb_expo(a_lo);
+        const float qh = hi_pe(b) * inv, ql = lo_pe(b) * inv;
+        const int ea = fb_expo(a_lo);
+        // Addends below half an ulp of the least binade that the sum can be in
+        // (it holds the first probability at least) add nothing, in any order
+        // and whatever the sum: it neither changes binade nor stops there. So
+        // masked tokens and the tail of an open nucleus need no replay, however
+        // many they are; every later bin is such a one too.
+        const bool none = __builtin_ldexpf(qh, 150 - max(ea, e_first)) < 0.5f;
+        // (the cut's bin: only where its tokens lie on both sides of the cut)
+        const bool split = static_cast<uint32_t>(b) == cut && qh >= minimum;
+        const bool kept = static_cast<uint32_t>(b) < cut || split;
+        if (static_cast<uint32_t>(b) == cut) sh.cut_elem = at + (split ? c : 0u);
+        if ((head && !none) || ((head || a_lo < tp) && kept)) {
+            const bool edge = none ? split : head || split || a_hi >= tp;
             uint32_t dc = 0, dw = 0;
-            const bool rc = edge || ea != fb_expo(a_hi) || ea == 0;
-            bool ex = rc || !fb_alike(ql, qh, ea, dc);
+            const bool rc = edge || (!none && (ea != fb_expo(a_hi) || ea == 0));
+            bool ex = rc || (!none && !fb_alike(ql, qh, ea, dc));
             int ew = 0;
             bool rw = false;
-            const double slack = c_hi * kFbDrift + (head ? __builtin_fabs(corr) : 0.0);
+            const double slack = c_hi * kFbDrift + (head && !none ? __builtin_fabs(corr) : 0.0);
             const double w_hi = c_hi + slack - W, w_lo = c_lo - slack - W1;
             if (w_hi > 0.0) {
                 ew = fb_expo(w_hi);
@@ -712,8 +723,8 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
         r.scal[kScSegs] = segs;
         r.scal[kScLarge] = 0u;
         // whether the list ends where the reference's sums do: the row's end,
-        // or the bin of the min-p cut
-        r.scal[kScCut] = elems == static_cast<uint32_t>(V) || (cut != 0xffffffffu && sh.cut_lo * (1.0 - kFbDrift) < tp) ? 1u : 0u;
+        // or the min-p cut
+        r.scal[kScCut] = elems == static_cast<uint32_t>(V) || elems == sh.cut_elem ? 1u : 0u;
         meta[kMetaItems] = G;
         meta[kMetaStatus] = kStatusOk;
     }
@@ -1238,7 +1249,9 @@ __device__ __forceinline__ void fb_draw(const DevArgs& a, int row, int parts, Dr
         int rc = 0;
         float s = q0;
         uint32_t keep = 1u;
-        if (good && limit > 1u) {
+        if (good && !(q0 < minimum) && q0 >= p.top_p && lc.n > 1 && lc.pos[1] == 1u && lc.elem[1] > 1u) {
+            keep = 2u;  // the first check comes after the second element, which adds nothing
+        } else if (good && !(q0 < minimum)) {
             const int hit = draw_chain<false>(lc, kc, limit, rc, s, p.top_p);
             if (hit < 0) good = false;
             else if (hit == 1) keep = lc.elem[rc] + (kc - lc.pos[rc]) + 1u;
