@@ -597,6 +597,9 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
         mass_lo = q_first;
         mass_hi = max(mass_hi, 2.0 * q_first);
     }
+    // (never more than the row holds: twice a first probability near 1 would
+    // put the whole tail into the draw's range)
+    mass_hi = min(mass_hi, max(all, q_first) * (1.0 + kFbDrift));
     const double u = static_cast<double>(a.uniforms[row]);
     // (a sum that top_p stops is the float itself: only one that ends at the cut
     // or the row's end has drifted)

@@ -186,7 +186,7 @@ def test_open_nuclei_take_no_sort(sampler, vocab, temperature, top_p):
 
 
 @pytest.mark.parametrize("vocab", [5003, 50257, W.VOCAB])
-@pytest.mark.parametrize("allowed", [300, 0.1])
+@pytest.mark.parametrize("allowed", [1, 2, 300, 0.1])
 @pytest.mark.parametrize("params", [dict(top_p=0.9), dict(top_p=1.0), dict(top_p=0.0), dict(top_p=2.0),
                                     dict(top_p=1.0, min_p=0.05), dict(top_p=0.9, min_p=1e-6)])
 def test_masked_rows_take_no_sort(sampler, vocab, allowed, params):
@@ -203,3 +203,16 @@ def test_masked_rows_take_no_sort(sampler, vocab, allowed, params):
     assert rows_left(sampler, 4) == []
     w.uniforms[:] = np.float32(1 - 2**-24)  # the last kept token, wherever it lies
     _check(sampler, w)
+
+
+@pytest.mark.parametrize("vocab", [5003, 32003, W.VOCAB])
+@pytest.mark.parametrize("first", [9.0, 14.0, 20.0, 30.0])
+@pytest.mark.parametrize("top_p", [0.95, 1.0])
+def test_one_probability_holds_the_nucleus(sampler, vocab, first, top_p):
+    # a confident row: its first probability reaches top_p, or nearly 1, alone
+    rng = np.random.default_rng(vocab)
+    x = (rng.standard_normal((6, vocab)) * 1.2).astype(np.float32)
+    x[:, 7] = first
+    u = np.array([0.0, 0.55, 0.8, 0.96, 0.9999, float(np.float32(1 - 2**-24))], np.float32)
+    _check(sampler, small_workload(f"confident-{vocab}", x, dict(temperature=0.7, top_k=0, top_p=top_p), uniforms=u))
+    assert [r for r in rows_left(sampler, 6) if r < 4] == []
