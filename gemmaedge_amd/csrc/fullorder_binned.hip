@@ -188,6 +188,12 @@ __device__ __forceinline__ void fb_stream_steps(const float* rowp, bool vec, int
     }
 }
 
+// The words that fo_left_kernel counts in, for any row of the call (one thread).
+__device__ __forceinline__ void fb_clear_left(const DevArgs& a, int row) {
+    fb_meta(a, row)[kMetaProgress] = 0u;
+    if (row == 0) fb_meta(a, row)[kMetaTicket] = 0u;
+}
+
 // Largest and smallest of one key per thread over the workgroup.
 __device__ __forceinline__ uint32_t fb_block_max(uint32_t v, uint32_t* s) {
     const uint32_t w = wave::max_u32(v);
@@ -1403,6 +1409,7 @@ __global__ __launch_bounds__(kFT) void fb_range_kernel(DevArgs a) {
 __global__ __launch_bounds__(kFT) void fb_exps_kernel(DevArgs a) {
     __shared__ ExpsShared sh;
     fb_exps(a, blockIdx.y, blockIdx.x, gridDim.x, sh);
+    if (blockIdx.x == 0 && threadIdx.x == 0) fb_clear_left(a, blockIdx.y);
 }
 template <int kPer>
 __global__ __launch_bounds__(kFT) void fb_plan_kernel(DevArgs a, int parts) {
@@ -1448,6 +1455,7 @@ __global__ __launch_bounds__(kFT) void fb_row_kernel(DevArgs a) {
     const int row = blockIdx.x;
     ge_sample_params p;
     uint32_t k;
+    if (threadIdx.x == 0) fb_clear_left(a, row);
     fb_range(a, row, 0, 1, sh.range);
     if (!fb_serves(a, row, p)) {  // (block-uniform) done rows are reported by the draw
         if (full_order_row(p, a.vocab, k) && row_done(a, row)) fb_draw<kFT>(a, row, 1, sh.draw);

@@ -19,7 +19,10 @@ enum : uint32_t {
     kMetaItems = 0, kMetaExtras = 1, kMetaNan = 2, kMetaStatus = 3,
     // sorted rows only: the top k's exps, from the sort kernel (their sum
     // as two words of a double, the lowest set bit, any NaN)
-    kMetaSumLo = 4, kMetaSumHi = 5, kMetaMinLsb = 6, kMetaAnyNan = 7
+    kMetaSumLo = 4, kMetaSumHi = 5, kMetaMinLsb = 6, kMetaAnyNan = 7,
+    // f32 calls: the tiles of a left row that are done, and (row 0) the next
+    // work item of fo_left_kernel; the sort-free kernels clear both
+    kMetaProgress = 8, kMetaTicket = 9
 };
 // kStatusToSort: a row left to the sort-based fallback pass (bf16: more
 // penalised ids than the extras hold; f32: not served without a sort);

@@ -663,28 +663,13 @@ __device__ __forceinline__ uint32_t digit_excl_scan(uint32_t v, uint32_t* scan, 
     return before + incl - v;
 }
 
+// One row by one workgroup.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void fo_sort_kernel(DevArgs a) {
-    __shared__ SortShared sh;
+__device__ __forceinline__ void sort_row(const DevArgs& a, int row, const ge_sample_params& p, uint32_t k, SortShared& sh) {
     const int tid = threadIdx.x;
     const int lane = __lane_id();
     const int wave = tid >> 6;
-    const int row = blockIdx.x;
     const int V = a.vocab;
-    const ge_sample_params p = params_of(a, row);
-    uint32_t k;
-    if (!full_order_row(p, V, k) || row_done(a, row)) return;  // done rows: fo_decide_kernel reports them
-    if (a.fo_fallback) {
-        // Only rows the first pass flagged (its status word, at the call
-        // row); the decide kernel of this pass skips the others.
-        const uint32_t st = a.fo_meta[static_cast<int64_t>(a.fo_row0 + row) * kMetaWords + kMetaStatus];
-        __syncthreads();  // every thread has read it before thread 0 may rewrite it below
-        if (st != kStatusToSort) {
-            if (tid == 0) a.fo_meta[static_cast<int64_t>(row) * kMetaWords + kMetaStatus] = kStatusSkip;
-            return;
-        }
-    }
-
     const T* rowp = static_cast<const T*>(a.logits) + static_cast<int64_t>(row) * a.row_stride;
     const int32_t* hist;
     int H;
@@ -962,6 +947,27 @@ __global__ __launch_bounds__(kThreads) void fo_sort_kernel(DevArgs a) {
     }
 }
 
+template <typename T>
+__global__ __launch_bounds__(kThreads) void fo_sort_kernel(DevArgs a) {
+    __shared__ SortShared sh;
+    const int tid = threadIdx.x;
+    const int row = blockIdx.x;
+    const ge_sample_params p = params_of(a, row);
+    uint32_t k;
+    if (!full_order_row(p, a.vocab, k) || row_done(a, row)) return;  // done rows: fo_decide_kernel reports them
+    if (a.fo_fallback) {
+        // Only rows the first pass flagged (its status word, at the call
+        // row); the decide kernel of this pass skips the others.
+        const uint32_t st = a.fo_meta[static_cast<int64_t>(a.fo_row0 + row) * kMetaWords + kMetaStatus];
+        __syncthreads();  // every thread has read it before thread 0 may rewrite it below
+        if (st != kStatusToSort) {
+            if (tid == 0) a.fo_meta[static_cast<int64_t>(row) * kMetaWords + kMetaStatus] = kStatusSkip;
+            return;
+        }
+    }
+    sort_row<T>(a, row, p, k, sh);
+}
+
 // ---- f32 rows over many workgroups: the same items, tile by tile -----------
 //
 // The sort above gives each row one workgroup; with few rows most of the GPU
@@ -977,7 +983,6 @@ __global__ __launch_bounds__(kThreads) void fo_sort_kernel(DevArgs a) {
 // output positions, the tiles' item counts and their certificate partials.
 
 constexpr int kSThreads = 256;
-constexpr int kSWaves = kSThreads / 64;
 constexpr int kSSteps = 16;                     // 64-key steps per wave per tile
 constexpr int kSTile = kSThreads * kSSteps;     // 4096 keys
 constexpr int kKThreads = 1024;                  // fs_keys_kernel's workgroup
@@ -1005,10 +1010,25 @@ __device__ __forceinline__ bool split_row_active(const DevArgs& a, int row, uint
     return full_order_row(p, a.vocab, k) && !row_done(a, row);
 }
 
+// What one tile leaves for others: plain accesses where each step is a kernel
+// of its own, agent-scope ones (which pass the caches that are not coherent
+// between the XCDs) where one launch takes every step (fo_left_kernel).
+template <bool kAgent, typename U>
+__device__ __forceinline__ U tile_ld(const U* p) {
+    if constexpr (kAgent) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else return *p;
+}
+template <bool kAgent, typename U>
+__device__ __forceinline__ void tile_st(U* p, U v) {
+    if constexpr (kAgent) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = v;
+}
+
 // Items before tile t: the sum of the tiles' item counts (one wave).
+template <bool kAgent>
 __device__ __forceinline__ uint32_t items_before(const uint32_t* bc, int t) {
     uint32_t s = 0;
-    for (int i = __lane_id(); i < t; i += 64) s += bc[i];
+    for (int i = __lane_id(); i < t; i += 64) s += tile_ld<kAgent>(bc + i);
     return wave::readlane(wave::incl_add(s), 63);
 }
 
@@ -1036,14 +1056,17 @@ __global__ __launch_bounds__(kSThreads) void fs_bitmap_kernel(DevArgs a) {
 //    the history (fs_bitmap_kernel is then not launched).
 // (1024 threads: 16 waves per CU hide the softcap's dependent latency, where
 // one wave per SIMD did not)
-__global__ __launch_bounds__(kKThreads) void fs_keys_kernel(DevArgs a, int fused) {
-    __shared__ uint32_t h[kDigits];
-    __shared__ uint32_t tbits[kSTile / 32];
-    const int t = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
-    uint32_t k;
-    ge_sample_params p;
-    if (!split_row_active(a, row, k, p)) return;
-    const int V = a.vocab, T = gridDim.x;
+struct KeysShared {
+    uint32_t h[kDigits];
+    uint32_t tbits[kSTile / 32];
+};
+template <bool kAgent>
+__device__ __forceinline__ void split_keys(const DevArgs& a, int t, int T, int row, const ge_sample_params& p, int fused,
+                                           KeysShared& sh) {
+    uint32_t* h = sh.h;
+    uint32_t* tbits = sh.tbits;
+    const int tid = threadIdx.x;
+    const int V = a.vocab;
     const int32_t* hist;
     int H;
     history_of(a, row, hist, H);
@@ -1083,22 +1106,31 @@ __global__ __launch_bounds__(kKThreads) void fs_keys_kernel(DevArgs a, int fused
             float f = softcap(x[u], p.softcap);
             if ((bw[u] >> (i & 31)) & 1u) f = penalize(f, p.repetition_penalty);
             const uint32_t s = ~order_key(f);
-            buf0[i] = s;
+            tile_st<kAgent>(buf0 + i, s);
             atomicAdd(&h[s & 255u], 1u);
         }
     }
     __syncthreads();
-    if (tid < kDigits) split_row(a, row, T).cnt[t * kDigits + tid] = h[tid];
+    if (tid < kDigits) tile_st<kAgent>(split_row(a, row, T).cnt + t * kDigits + tid, h[tid]);
+}
+
+__global__ __launch_bounds__(kKThreads) void fs_keys_kernel(DevArgs a, int fused) {
+    __shared__ KeysShared sh;
+    uint32_t k;
+    ge_sample_params p;
+    if (split_row_active(a, blockIdx.y, k, p)) split_keys<false>(a, blockIdx.x, gridDim.x, blockIdx.y, p, fused, sh);
 }
 
 // 3a. The tile's count of each digit of pass `shift` (passes after the first).
-__global__ __launch_bounds__(kKThreads) void fs_count_kernel(DevArgs a, int shift, int src_is_buf1) {  // (1024 threads)
-    __shared__ uint32_t h[kDigits];
-    const int t = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
-    uint32_t k;
-    ge_sample_params p;
-    if (!split_row_active(a, row, k, p)) return;
-    const int V = a.vocab, T = gridDim.x;
+struct CountShared {
+    uint32_t h[kDigits];
+};
+template <bool kAgent>
+__device__ __forceinline__ void split_count(const DevArgs& a, int t, int T, int row, int shift, int src_is_buf1,
+                                            CountShared& sh) {
+    uint32_t* h = sh.h;
+    const int tid = threadIdx.x;
+    const int V = a.vocab;
     const uint32_t* src = src_is_buf1 ? a.fo_pre + static_cast<int64_t>(row) * a.fo_items_stride
                                       : reinterpret_cast<const uint32_t*>(a.fo_aux) + static_cast<int64_t>(row) * a.fo_items_stride;
     if (tid < kDigits) h[tid] = 0u;
@@ -1107,7 +1139,7 @@ __global__ __launch_bounds__(kKThreads) void fs_count_kernel(DevArgs a, int shif
 #pragma unroll
     for (int u = 0; u < kKSteps; ++u) {
         const int i = t * kSTile + u * kKThreads + tid;
-        kv[u] = src[min(i, V - 1)];  // clamped: keys past V unused
+        kv[u] = tile_ld<kAgent>(src + min(i, V - 1));  // clamped: keys past V unused
     }
 #pragma unroll
     for (int u = 0; u < kKSteps; ++u) {
@@ -1115,40 +1147,56 @@ __global__ __launch_bounds__(kKThreads) void fs_count_kernel(DevArgs a, int shif
         if (i < V) atomicAdd(&h[(kv[u] >> shift) & 255u], 1u);
     }
     __syncthreads();
-    if (tid < kDigits) split_row(a, row, T).cnt[t * kDigits + tid] = h[tid];
+    if (tid < kDigits) tile_st<kAgent>(split_row(a, row, T).cnt + t * kDigits + tid, h[tid]);
+}
+
+__global__ __launch_bounds__(kKThreads) void fs_count_kernel(DevArgs a, int shift, int src_is_buf1) {  // (1024 threads)
+    __shared__ CountShared sh;
+    uint32_t k;
+    ge_sample_params p;
+    if (split_row_active(a, blockIdx.y, k, p)) split_count<false>(a, blockIdx.x, gridDim.x, blockIdx.y, shift, src_is_buf1, sh);
 }
 
 // 3b. Output position of each (digit, tile) group: digits in order, tiles in
 //     order inside a digit (a stable pass). In place over the counts; thread
 //     d walks its digit's counts down the tiles, 64 loads in flight, a wave's
-//     loads of one tile on consecutive words.
-__global__ __launch_bounds__(kSThreads) void fs_scan_kernel(DevArgs a, int T) {
-    __shared__ uint32_t scan[kSWaves];
+//     loads of one tile on consecutive words. (Threads past the digits only
+//     meet the barrier.)
+struct ScanShared {
+    uint32_t scan[kKThreads / 64];
+};
+template <bool kAgent>
+__device__ __forceinline__ void split_scan(const DevArgs& a, int T, int row, ScanShared& sh) {
     constexpr int kB = 64;
-    const int row = blockIdx.x, tid = threadIdx.x;
-    uint32_t k;
-    ge_sample_params p;
-    if (!split_row_active(a, row, k, p)) return;
-    uint32_t* c = split_row(a, row, T).cnt + tid;
+    const int tid = threadIdx.x;
+    const int tiles = tid < kDigits ? T : 0;
+    uint32_t* c = split_row(a, row, T).cnt + min(tid, kDigits - 1);
     uint32_t total = 0;
-    for (int t0 = 0; t0 < T; t0 += kB) {
+    for (int t0 = 0; t0 < tiles; t0 += kB) {
         uint32_t v[kB];
 #pragma unroll
-        for (int u = 0; u < kB; ++u) v[u] = c[min(t0 + u, T - 1) * kDigits];
+        for (int u = 0; u < kB; ++u) v[u] = tile_ld<kAgent>(c + min(t0 + u, T - 1) * kDigits);
 #pragma unroll
         for (int u = 0; u < kB; ++u) total += t0 + u < T ? v[u] : 0u;
     }
-    uint32_t run = digit_excl_scan(total, scan, tid);
-    for (int t0 = 0; t0 < T; t0 += kB) {
+    uint32_t run = digit_excl_scan(total, sh.scan, tid);
+    for (int t0 = 0; t0 < tiles; t0 += kB) {
         uint32_t v[kB];
 #pragma unroll
-        for (int u = 0; u < kB; ++u) v[u] = c[min(t0 + u, T - 1) * kDigits];
+        for (int u = 0; u < kB; ++u) v[u] = tile_ld<kAgent>(c + min(t0 + u, T - 1) * kDigits);
 #pragma unroll
         for (int u = 0; u < kB; ++u) {
-            if (t0 + u < T) c[(t0 + u) * kDigits] = run;
+            if (t0 + u < T) tile_st<kAgent>(c + (t0 + u) * kDigits, run);
             run += t0 + u < T ? v[u] : 0u;
         }
     }
+}
+
+__global__ __launch_bounds__(kSThreads) void fs_scan_kernel(DevArgs a, int T) {
+    __shared__ ScanShared sh;
+    uint32_t k;
+    ge_sample_params p;
+    if (split_row_active(a, blockIdx.x, k, p)) split_scan<false>(a, T, blockIdx.x, sh);
 }
 
 // 3c. The stable scatter of tile t by the digit at `shift`: ranks among the
@@ -1159,19 +1207,25 @@ __global__ __launch_bounds__(kSThreads) void fs_scan_kernel(DevArgs a, int T) {
 //     tiles' counts itself, as fs_scan_kernel would (which then is not
 //     launched): every tile of a row reads the row's counts.
 // (1024 threads, as fs_keys_kernel: threads tid < 256 hold the per-digit work)
-__global__ __launch_bounds__(kKThreads) void fs_scatter_kernel(DevArgs a, int shift, int src_is_buf1, int fused) {
+struct ScatterShared {
+    uint32_t staged[kSTile];
+    uint32_t wc[kKThreads / 64][kDigits];
+    uint32_t toff[kDigits];
+    uint32_t gb[kDigits];
+    uint32_t scan[kKThreads / 64];
+};
+template <bool kAgent>
+__device__ __forceinline__ void split_scatter(const DevArgs& a, int t, int T, int row, int shift, int src_is_buf1, int fused,
+                                              ScatterShared& sh) {
     constexpr int kKWaves = kKThreads / 64;
-    __shared__ uint32_t staged[kSTile];
-    __shared__ uint32_t wc[kKWaves][kDigits];
-    __shared__ uint32_t toff[kDigits];
-    __shared__ uint32_t gb[kDigits];
-    __shared__ uint32_t scan[kKWaves];
-    const int t = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+    uint32_t* staged = sh.staged;
+    auto& wc = sh.wc;
+    uint32_t* toff = sh.toff;
+    uint32_t* gb = sh.gb;
+    uint32_t* scan = sh.scan;
+    const int tid = threadIdx.x;
     const int lane = __lane_id(), wave = tid >> 6;
-    uint32_t k;
-    ge_sample_params p;
-    if (!split_row_active(a, row, k, p)) return;
-    const int V = a.vocab, T = gridDim.x;
+    const int V = a.vocab;
     uint32_t* b0 = reinterpret_cast<uint32_t*>(a.fo_aux) + static_cast<int64_t>(row) * a.fo_items_stride;
     uint32_t* b1 = a.fo_pre + static_cast<int64_t>(row) * a.fo_items_stride;
     const uint32_t* src = src_is_buf1 ? b1 : b0;
@@ -1180,7 +1234,7 @@ __global__ __launch_bounds__(kKThreads) void fs_scatter_kernel(DevArgs a, int sh
 #pragma unroll
     for (int u = 0; u < kKSteps; ++u) {
         const int i = t * kSTile + wave * (64 * kKSteps) + u * 64 + lane;
-        key[u] = src[min(i, V - 1)];  // clamped: keys past V unused
+        key[u] = tile_ld<kAgent>(src + min(i, V - 1));  // clamped: keys past V unused
     }
     for (int d = lane; d < kDigits; d += 64) wc[wave][d] = 0u;  // only this wave uses its row
     if (fused) {
@@ -1202,7 +1256,7 @@ __global__ __launch_bounds__(kKThreads) void fs_scatter_kernel(DevArgs a, int sh
         const uint32_t ex = digit_excl_scan(total, scan, tid);  // (scan[] is read again after a barrier)
         if (tid < kDigits) gb[tid] = ex + part;
     } else if (tid < kDigits) {
-        gb[tid] = split_row(a, row, T).cnt[t * kDigits + tid];
+        gb[tid] = tile_ld<kAgent>(split_row(a, row, T).cnt + t * kDigits + tid);
     }
     const uint64_t below = (1ull << lane) - 1ull;
     uint32_t lr[kKSteps];
@@ -1250,33 +1304,43 @@ __global__ __launch_bounds__(kKThreads) void fs_scatter_kernel(DevArgs a, int sh
         if (q < nt) {
             const uint32_t kv = staged[q];
             const uint32_t d = (kv >> shift) & 255u;
-            dst[gb[d] + static_cast<uint32_t>(q) - toff[d]] = kv;
+            tile_st<kAgent>(dst + (gb[d] + static_cast<uint32_t>(q) - toff[d]), kv);
         }
     }
 }
 
+__global__ __launch_bounds__(kKThreads) void fs_scatter_kernel(DevArgs a, int shift, int src_is_buf1, int fused) {
+    __shared__ ScatterShared sh;
+    uint32_t k;
+    ge_sample_params p;
+    if (split_row_active(a, blockIdx.y, k, p))
+        split_scatter<false>(a, blockIdx.x, gridDim.x, blockIdx.y, shift, src_is_buf1, fused, sh);
+}
+
 // Item boundaries of the sorted keys: position i starts an item when i == 0
 // or its key differs from position i - 1's.
+template <bool kAgent>
 __device__ __forceinline__ bool is_boundary(const uint32_t* s, int i, int V, uint32_t kv) {
-    return i < V && (i == 0 || kv != s[i - 1]);
+    return i < V && (i == 0 || kv != tile_ld<kAgent>(s + i - 1));
 }
 
 // 4a. Items starting in tile t.
-__global__ __launch_bounds__(kKThreads) void fs_bounds_kernel(DevArgs a) {  // (1024 threads)
+struct BoundsShared {
+    uint32_t red[kKThreads / 64];
+};
+template <bool kAgent>
+__device__ __forceinline__ void split_bounds(const DevArgs& a, int t, int T, int row, BoundsShared& sh) {
     constexpr int kKWaves = kKThreads / 64;
-    __shared__ uint32_t red[kKWaves];
-    const int t = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
-    uint32_t k;
-    ge_sample_params p;
-    if (!split_row_active(a, row, k, p)) return;
-    const int V = a.vocab, T = gridDim.x;
+    uint32_t* red = sh.red;
+    const int tid = threadIdx.x;
+    const int V = a.vocab;
     const uint32_t* s = reinterpret_cast<const uint32_t*>(a.fo_aux) + static_cast<int64_t>(row) * a.fo_items_stride;
     uint32_t n = 0;
 #pragma unroll
     for (int u = 0; u < kKSteps; ++u) {
         const int i = t * kSTile + u * kKThreads + tid;
-        const uint32_t kv = s[min(i, V - 1)];  // clamped: is_boundary checks i < V
-        n += is_boundary(s, i, V, kv) ? 1u : 0u;
+        const uint32_t kv = tile_ld<kAgent>(s + min(i, V - 1));  // clamped: is_boundary checks i < V
+        n += is_boundary<kAgent>(s, i, V, kv) ? 1u : 0u;
     }
     n = wave::readlane(wave::incl_add(n), 63);
     if (__lane_id() == 0) red[tid >> 6] = n;
@@ -1284,29 +1348,38 @@ __global__ __launch_bounds__(kKThreads) void fs_bounds_kernel(DevArgs a) {  // (
     if (tid == 0) {
         uint32_t c = 0;
         for (int w = 0; w < kKWaves; ++w) c += red[w];
-        split_row(a, row, T).bc[t] = c;
+        tile_st<kAgent>(split_row(a, row, T).bc + t, c);
     }
+}
+
+__global__ __launch_bounds__(kKThreads) void fs_bounds_kernel(DevArgs a) {  // (1024 threads)
+    __shared__ BoundsShared sh;
+    uint32_t k;
+    ge_sample_params p;
+    if (split_row_active(a, blockIdx.y, k, p)) split_bounds<false>(a, blockIdx.x, gridDim.x, blockIdx.y, sh);
 }
 
 // 4b. Each item's first element into pre (buf1), in position order, and its
 //     value into the high word of its items entry (4c adds the count); the
 //     last tile also writes pre[G] = V.
-__global__ __launch_bounds__(kKThreads) void fs_istart_kernel(DevArgs a) {  // (1024 threads)
+struct IstartShared {
+    uint32_t scan[kKThreads / 64];
+    uint32_t base_s;
+};
+template <bool kAgent>
+__device__ __forceinline__ void split_istart(const DevArgs& a, int t, int T, int row, IstartShared& sh) {
     constexpr int kKWaves = kKThreads / 64;
-    __shared__ uint32_t scan[kKWaves];
-    __shared__ uint32_t base_s;
-    const int t = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+    uint32_t* scan = sh.scan;
+    uint32_t& base_s = sh.base_s;
+    const int tid = threadIdx.x;
     const int lane = __lane_id(), wave = tid >> 6;
-    uint32_t k;
-    ge_sample_params p;
-    if (!split_row_active(a, row, k, p)) return;
-    const int V = a.vocab, T = gridDim.x;
+    const int V = a.vocab;
     const SplitRow sr = split_row(a, row, T);
     const uint32_t* s = reinterpret_cast<const uint32_t*>(a.fo_aux) + static_cast<int64_t>(row) * a.fo_items_stride;
     uint32_t* istart = a.fo_pre + static_cast<int64_t>(row) * a.fo_items_stride;
     uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
     if (wave == 0) {
-        const uint32_t b = items_before(sr.bc, t);
+        const uint32_t b = items_before<kAgent>(sr.bc, t);
         if (lane == 0) base_s = b;
     }
     // wave w owns positions [w * 256, (w + 1) * 256) of the tile
@@ -1316,12 +1389,12 @@ __global__ __launch_bounds__(kKThreads) void fs_istart_kernel(DevArgs a) {  // (
 #pragma unroll
     for (int u = 0; u < kKSteps; ++u) {
         const int i = t * kSTile + wave * (64 * kKSteps) + u * 64 + lane;
-        kv[u] = s[min(i, V - 1)];  // clamped: is_boundary checks i < V
+        kv[u] = tile_ld<kAgent>(s + min(i, V - 1));  // clamped: is_boundary checks i < V
     }
 #pragma unroll
     for (int u = 0; u < kKSteps; ++u) {
         const int i = t * kSTile + wave * (64 * kKSteps) + u * 64 + lane;
-        bnd[u] = is_boundary(s, i, V, kv[u]);
+        bnd[u] = is_boundary<kAgent>(s, i, V, kv[u]);
         nb += static_cast<uint32_t>(__popcll(__ballot(bnd[u])));
     }
     if (lane == 0) scan[wave] = nb;
@@ -1336,16 +1409,23 @@ __global__ __launch_bounds__(kKThreads) void fs_istart_kernel(DevArgs a) {  // (
         if (bnd[u]) {
             const uint32_t jj = j + static_cast<uint32_t>(__popcll(m & below));
             const uint32_t key = ~kv[u];
-            istart[jj] = static_cast<uint32_t>(i);
-            items[jj] = static_cast<uint64_t>(key == kKeyNaN ? 0x7fc00000u : f2u(key_value(key))) << 32;
+            tile_st<kAgent>(istart + jj, static_cast<uint32_t>(i));
+            tile_st<kAgent>(items + jj, static_cast<uint64_t>(key == kKeyNaN ? 0x7fc00000u : f2u(key_value(key))) << 32);
         }
         j += static_cast<uint32_t>(__popcll(m));
     }
     if (t == T - 1 && tid == 0) {
         uint32_t c = base_s;
         for (int w = 0; w < kKWaves; ++w) c += scan[w];
-        istart[c] = static_cast<uint32_t>(V);
+        tile_st<kAgent>(istart + c, static_cast<uint32_t>(V));
     }
+}
+
+__global__ __launch_bounds__(kKThreads) void fs_istart_kernel(DevArgs a) {  // (1024 threads)
+    __shared__ IstartShared sh;
+    uint32_t k;
+    ge_sample_params p;
+    if (split_row_active(a, blockIdx.y, k, p)) split_istart<false>(a, blockIdx.x, gridDim.x, blockIdx.y, sh);
 }
 
 // 4c. The items that start in tile t: each one's count (from the next
@@ -1354,30 +1434,34 @@ __global__ __launch_bounds__(kKThreads) void fs_istart_kernel(DevArgs a) {  // (
 //     item's value), and the tile's part of the certificate of the top k's
 //     double sum: the sum, the lowest set bit, any NaN. aux held the sorted
 //     keys, which 4b was the last to read.
-__global__ __launch_bounds__(kKThreads) void fs_exps_kernel(DevArgs a) {  // (1024 threads, as fs_keys_kernel)
+struct SplitExpsShared {
+    uint32_t base_s;
+    double dred[kKThreads / 64];
+    int ired[kKThreads / 64];
+    uint32_t ured[kKThreads / 64];
+};
+template <bool kAgent>
+__device__ __forceinline__ void split_exps(const DevArgs& a, int t, int T, int row, const ge_sample_params& p, uint32_t k,
+                                           SplitExpsShared& sh) {
     constexpr int kKWaves = kKThreads / 64;
-    __shared__ uint32_t base_s;
-    __shared__ double dred[kKWaves];
-    __shared__ int ired[kKWaves];
-    __shared__ uint32_t ured[kKWaves];
-    const int t = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+    uint32_t& base_s = sh.base_s;
+    double* dred = sh.dred;
+    int* ired = sh.ired;
+    uint32_t* ured = sh.ured;
+    const int tid = threadIdx.x;
     const int lane = __lane_id(), wave = tid >> 6;
-    uint32_t k;
-    ge_sample_params p;
-    if (!split_row_active(a, row, k, p)) return;
-    const int T = gridDim.x;
     const SplitRow sr = split_row(a, row, T);
     const uint32_t* istart = a.fo_pre + static_cast<int64_t>(row) * a.fo_items_stride;
     uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
     float* aux = a.fo_aux + static_cast<int64_t>(row) * a.fo_items_stride;
     if (wave == 0) {
-        const uint32_t b = items_before(sr.bc, t);
+        const uint32_t b = items_before<kAgent>(sr.bc, t);
         if (lane == 0) base_s = b;
     }
     __syncthreads();
-    const float vmax = u2f(static_cast<uint32_t>(items[0] >> 32));
+    const float vmax = u2f(static_cast<uint32_t>(tile_ld<kAgent>(items) >> 32));
     const float inv_temp = 1.0f / p.temperature;
-    const uint32_t j0 = base_s, nj = sr.bc[t];
+    const uint32_t j0 = base_s, nj = tile_ld<kAgent>(sr.bc + t);
     double S = 0.0;
     int minlsb = INT_MAX;
     bool nan = false;
@@ -1387,9 +1471,9 @@ __global__ __launch_bounds__(kKThreads) void fs_exps_kernel(DevArgs a) {  // (10
 #pragma unroll
         for (int u = 0; u < kKSteps; ++u) {  // nj <= kSTile; clamped indices, no conditional load
             const uint32_t q = min(static_cast<uint32_t>(u * kKThreads + tid), nj - 1u);
-            itv[u] = items[j0 + q];
-            stv[u] = istart[j0 + q];
-            env[u] = istart[j0 + q + 1];
+            itv[u] = tile_ld<kAgent>(items + j0 + q);
+            stv[u] = tile_ld<kAgent>(istart + j0 + q);
+            env[u] = tile_ld<kAgent>(istart + j0 + q + 1);
         }
     }
 #pragma unroll
@@ -1398,9 +1482,9 @@ __global__ __launch_bounds__(kKThreads) void fs_exps_kernel(DevArgs a) {  // (10
         if (q < nj) {
             const uint32_t n = env[u] - stv[u];
             const uint32_t vb = static_cast<uint32_t>(itv[u] >> 32);
-            items[j0 + q] = (static_cast<uint64_t>(vb) << 32) | n;
+            tile_st<kAgent>(items + j0 + q, (static_cast<uint64_t>(vb) << 32) | n);
             const float pe = expf_glibc((u2f(vb) - vmax) * inv_temp);
-            aux[j0 + q] = pe;
+            tile_st<kAgent>(aux + j0 + q, pe);
             const uint32_t nk = top_k_count(stv[u], n, k);
             if (nk) {
                 if (pe != pe) nan = true;
@@ -1431,29 +1515,35 @@ __global__ __launch_bounds__(kKThreads) void fs_exps_kernel(DevArgs a) {  // (10
         }
         const uint64_t sb = __builtin_bit_cast(uint64_t, Sp);
         uint32_t* pt = sr.part + 4 * t;
-        pt[0] = static_cast<uint32_t>(sb);
-        pt[1] = static_cast<uint32_t>(sb >> 32);
-        pt[2] = static_cast<uint32_t>(ml);
-        pt[3] = nn;
+        tile_st<kAgent>(pt + 0, static_cast<uint32_t>(sb));
+        tile_st<kAgent>(pt + 1, static_cast<uint32_t>(sb >> 32));
+        tile_st<kAgent>(pt + 2, static_cast<uint32_t>(ml));
+        tile_st<kAgent>(pt + 3, nn);
     }
 }
 
-// 4d. The row's meta words, as fo_sort_kernel writes them.
-__global__ __launch_bounds__(64) void fs_meta_kernel(DevArgs a, int T) {
-    const int row = blockIdx.x, lane = __lane_id();
+__global__ __launch_bounds__(kKThreads) void fs_exps_kernel(DevArgs a) {  // (1024 threads, as fs_keys_kernel)
+    __shared__ SplitExpsShared sh;
     uint32_t k;
     ge_sample_params p;
-    if (!split_row_active(a, row, k, p)) return;
+    if (split_row_active(a, blockIdx.y, k, p)) split_exps<false>(a, blockIdx.x, gridDim.x, blockIdx.y, p, k, sh);
+}
+
+// 4d. The row's meta words, as fo_sort_kernel writes them (one wave).
+template <bool kAgent>
+__device__ __forceinline__ void split_meta(const DevArgs& a, int T, int row) {
+    const int lane = __lane_id();
     const SplitRow sr = split_row(a, row, T);
     double S = 0.0;
     int ml = INT_MAX;
     uint32_t nn = 0, G = 0;
     for (int t = lane; t < T; t += 64) {
         const uint32_t* pt = sr.part + 4 * t;
-        S += __builtin_bit_cast(double, (static_cast<uint64_t>(pt[1]) << 32) | pt[0]);
-        ml = min(ml, static_cast<int>(pt[2]));
-        nn |= pt[3];
-        G += sr.bc[t];
+        const uint32_t lo = tile_ld<kAgent>(pt + 0), hi = tile_ld<kAgent>(pt + 1);
+        S += __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+        ml = min(ml, static_cast<int>(tile_ld<kAgent>(pt + 2)));
+        nn |= tile_ld<kAgent>(pt + 3);
+        G += tile_ld<kAgent>(sr.bc + t);
     }
     S = wave::sum_f64(S);
     ml = wave::min_i32(ml);
@@ -1462,18 +1552,23 @@ __global__ __launch_bounds__(64) void fs_meta_kernel(DevArgs a, int T) {
     if (lane == 0) {
         const uint64_t* items = a.fo_items + static_cast<int64_t>(row) * a.fo_items_stride;
         const uint32_t* istart = a.fo_pre + static_cast<int64_t>(row) * a.fo_items_stride;
-        const bool last_nan = static_cast<uint32_t>(items[G - 1] >> 32) == 0x7fc00000u;
+        const bool last_nan = static_cast<uint32_t>(tile_ld<kAgent>(items + G - 1) >> 32) == 0x7fc00000u;
         uint32_t* meta = a.fo_meta + static_cast<int64_t>(row) * kMetaWords;
         const uint64_t sb = __builtin_bit_cast(uint64_t, S);
-        meta[kMetaSumLo] = static_cast<uint32_t>(sb);
-        meta[kMetaSumHi] = static_cast<uint32_t>(sb >> 32);
-        meta[kMetaMinLsb] = static_cast<uint32_t>(ml);
-        meta[kMetaAnyNan] = nn;
-        meta[kMetaItems] = G;
+        tile_st<kAgent>(meta + kMetaSumLo, static_cast<uint32_t>(sb));
+        tile_st<kAgent>(meta + kMetaSumHi, static_cast<uint32_t>(sb >> 32));
+        tile_st<kAgent>(meta + kMetaMinLsb, static_cast<uint32_t>(ml));
+        tile_st<kAgent>(meta + kMetaAnyNan, nn);
+        tile_st<kAgent>(meta + kMetaItems, G);
         meta[kMetaExtras] = 0;
-        meta[kMetaNan] = last_nan ? static_cast<uint32_t>(a.vocab) - istart[G - 1] : 0u;
-        meta[kMetaStatus] = kStatusOk;
+        meta[kMetaNan] = last_nan ? static_cast<uint32_t>(a.vocab) - tile_ld<kAgent>(istart + G - 1) : 0u;
+        tile_st<kAgent>(meta + kMetaStatus, static_cast<uint32_t>(a.fo_fallback ? kStatusFallback : kStatusOk));
     }
+}
+__global__ __launch_bounds__(64) void fs_meta_kernel(DevArgs a, int T) {
+    uint32_t k;
+    ge_sample_params p;
+    if (split_row_active(a, blockIdx.x, k, p)) split_meta<false>(a, T, blockIdx.x);
 }
 
 // ---- kernel 2: probabilities, exact chains, token ----------------------------
@@ -1733,6 +1828,18 @@ __device__ __forceinline__ bool den_certified(const uint32_t* meta, double& S, u
 // S plus one (the two differ by far less than a binade).
 __device__ __forceinline__ int den_top_binade(double S) { return exp_of(S) + 1; }
 
+// Whether a row sorted in this launch has a denominator to replay (agent-scope
+// loads: another workgroup wrote the meta words).
+__device__ __forceinline__ bool den_open(const DevArgs& a, int row) {
+    uint32_t k;
+    if (!full_order_row(params_of(a, row), a.vocab, k) || k <= 1u) return false;
+    uint32_t meta[kMetaWords];
+#pragma unroll
+    for (int i = kMetaSumLo; i <= kMetaAnyNan; ++i) meta[i] = ld_l2(a.fo_meta + static_cast<int64_t>(row) * kMetaWords + i);
+    double S;
+    return !den_certified(meta, S, k, a.vocab);
+}
+
 // Whether part `part` (tile * kMapSub + p) of row `row` needs its maps: a
 // sorted row of this pass whose sum does not certify, with items in the part.
 __device__ __forceinline__ bool map_part_needed(const DevArgs& a, int row, int part) {
@@ -1751,6 +1858,7 @@ __device__ __forceinline__ bool map_part_needed(const DevArgs& a, int row, int p
 // a binade below a lower bound of the sum before the part gets a saturated
 // map (the decide kernel then replays).
 __device__ __forceinline__ void map_part(const DevArgs& a, int row, int part, uint64_t (&wmap)[2][kMapThreads / 64]) {
+    // (called by kMapThreads threads or more)
     const int tid = threadIdx.x;
     const int lane = __lane_id();
     const int wave = tid >> 6;
@@ -1792,7 +1900,7 @@ __device__ __forceinline__ void map_part(const DevArgs& a, int row, int part, ui
 #pragma unroll
     for (int j = 0; j < kMapPer; ++j) ab[j] = f2u(aux[min(ib + j, G - 1)]);
     const int b = bhi - (kMapBins - 1) + slot;
-    const bool live = b >= blo && b >= 0;  // (uniform in the group)
+    const bool live = slot < kMapBins && b >= blo && b >= 0;  // (uniform in the group; no slot: threads past them)
     if (live) {
         const int uexp = b - 52;
         DMap f{0, 0};
@@ -1813,7 +1921,7 @@ __device__ __forceinline__ void map_part(const DevArgs& a, int row, int part, ui
         }
     }
     __syncthreads();
-    if (gt == 0) {
+    if (gt == 0 && slot < kMapBins) {
         DMap tot{kMapCap, kMapCap};
         if (live) {
             tot = DMap{0, 0};
@@ -1845,6 +1953,170 @@ __global__ __launch_bounds__(kMapThreads) void fo_denmap_kernel(DevArgs a) {
         const int j = __ffsll(static_cast<unsigned long long>(todo)) - 1;
         todo &= todo - 1ull;
         map_part(a, static_cast<int>(blockIdx.y) + j * static_cast<int>(gridDim.y), part, wmap);
+    }
+}
+
+// ---- rows that the sort-free path leaves --------------------------------------
+//
+// fullorder_binned.hip serves nearly every f32 row with k = V; the host cannot
+// tell whether a call has a row that it left (or, with per-row parameters, one
+// with 1024 < k < V). This one launch finds those rows and takes them through
+// the many-workgroup sort above. (Launched as kernels of their own, its 14
+// steps cost every call about 25 us, against 5 for this launch without a row.)
+//
+// The steps' tiles are work items in one order, step by step, rows in order
+// inside a step. A workgroup takes the next item from a counter, waits until
+// the row's previous step is complete, works, and counts the tile in the
+// row's progress word. An item waits only for items before it, and those
+// have been taken by workgroups that run: whatever number of workgroups is
+// resident, the first unfinished item never waits, so every wait ends. (The
+// waits are bounded all the same: kLeftSpins.) The last tile of a step that a
+// row-wide step follows (the scan of the counts, the meta words) does that too.
+//
+// What one workgroup leaves for another goes through agent-scope accesses;
+// fences that write back and invalidate the L2 at each item took 200 us for one
+// row and 6,000 for 64. Measured so, rows of V = 262,144: one 100 us, 64 1,110; of
+// V = 50,257: 64 260. With one workgroup per row (fo_sort_kernel's body) any
+// number up to 256 takes 1,450 and 300: more than kLeftTiledRows rows do that.
+constexpr uint32_t kLeftSpins = 1u << 22;  // about 4 s of polling
+constexpr int kLeftSteps = 12;
+constexpr int kLeftTiledRows = 64;
+constexpr int kLeftMasks = 16;  // rows of a launch at most: 64 each
+static_assert(kThreads == kKThreads, "sort_row and the tiles share the workgroup");
+// Row-wide steps done before step s begins: a scan after each count, then the meta words.
+__device__ __forceinline__ uint32_t left_wide(int s) {
+    return static_cast<uint32_t>(s == 0 ? 0 : s >= kLeftSteps - 1 ? 5 : min((s + 1) / 2, 4));
+}
+struct LeftShared {
+    union {
+        KeysShared keys;
+        CountShared count;
+        ScanShared scan;
+        ScatterShared scatter;
+        BoundsShared bounds;
+        IstartShared istart;
+        SplitExpsShared exps;
+        SortShared sort;
+        uint64_t wmap[2][kMapThreads / 64];
+    };
+    uint64_t mask[kLeftMasks];
+    uint32_t rows[kLeftTiledRows];
+    uint32_t item, go;
+    __device__ LeftShared() {}
+};
+__device__ __forceinline__ bool row_left(const DevArgs& a, int row) {
+    uint32_t k;
+    ge_sample_params p;
+    // (a row this kernel has sorted already carries kStatusFallback)
+    return row < a.rows && split_row_active(a, row, k, p) &&
+           ld_l2(a.fo_meta + static_cast<int64_t>(row) * kMetaWords + kMetaStatus) != kStatusOk;
+}
+// The maps of parts [part0, part1), if the row's denominator needs them
+// (block-uniform). Few rows do: they alone pay for making the other
+// workgroups' stores visible to the maps' plain loads.
+__device__ __forceinline__ void left_maps(const DevArgs& a, int row, int part0, int part1, LeftShared& sh) {
+    if (!a.fo_maps || !den_open(a, row)) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    for (int part = part0; part < part1; ++part)
+        if (map_part_needed(a, row, part)) map_part(a, row, part, sh.wmap);
+}
+
+__global__ __launch_bounds__(kKThreads) void fo_left_kernel(DevArgs a) {
+    __shared__ LeftShared sh;
+    const int tid = threadIdx.x, lane = __lane_id(), wave = tid >> 6;
+    {
+        const uint64_t m = __ballot(row_left(a, tid));
+        if (lane == 0) sh.mask[wave] = m;
+    }
+    __syncthreads();
+    uint32_t n = 0, before = 0;
+    for (int w = 0; w < kLeftMasks; ++w) {
+        if (w < wave) before += static_cast<uint32_t>(__popcll(sh.mask[w]));
+        n += static_cast<uint32_t>(__popcll(sh.mask[w]));
+    }
+    if (n == 0u) return;
+    const int T = fo_split_tiles(a.vocab);
+    uint32_t k;
+    ge_sample_params p;
+    if (n > static_cast<uint32_t>(kLeftTiledRows)) {
+        for (int row = blockIdx.x; row < a.rows; row += gridDim.x) {
+            if (((sh.mask[row >> 6] >> (row & 63)) & 1ull) == 0ull) continue;
+            (void)split_row_active(a, row, k, p);
+            __syncthreads();
+            sort_row<float>(a, row, p, k, sh.sort);
+            stores_done_barrier();
+            left_maps(a, row, 0, T * kMapSub, sh);
+        }
+        return;
+    }
+    {
+        const uint64_t m = sh.mask[wave];
+        if ((m >> lane) & 1ull) sh.rows[before + static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)))] = static_cast<uint32_t>(tid);
+    }
+    uint32_t* ticket = a.fo_meta + kMetaTicket;
+    const uint32_t per = n * static_cast<uint32_t>(T);
+    const uint32_t total = per * static_cast<uint32_t>(kLeftSteps);
+    if (blockIdx.x >= per) return;  // (more would only poll)
+    for (;;) {
+        __syncthreads();  // the item before is done with the shared words
+        if (tid == 0) sh.item = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        const uint32_t item = sh.item;
+        if (item >= total) return;
+        const int step = static_cast<int>(item / per);
+        const uint32_t rem = item - static_cast<uint32_t>(step) * per;
+        const int row = static_cast<int>(sh.rows[rem / static_cast<uint32_t>(T)]);
+        const int t = static_cast<int>(rem % static_cast<uint32_t>(T));
+        uint32_t* progress = a.fo_meta + static_cast<int64_t>(row) * kMetaWords + kMetaProgress;
+        const uint32_t need = static_cast<uint32_t>(step * T) + left_wide(step);
+        if (step > 0) {
+            if (tid == 0) {
+                uint32_t it = 0;
+                while (ld_l2(progress) < need && it < kLeftSpins) {
+                    ++it;
+                    __builtin_amdgcn_s_sleep(1);
+                }
+                sh.go = it < kLeftSpins ? 1u : 0u;
+                // no workgroup takes another item (the row keeps kStatusToSort,
+                // which fo_decide_kernel reports)
+                if (it >= kLeftSpins) __hip_atomic_store(ticket, 0x80000000u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            __syncthreads();
+            if (sh.go == 0u) return;
+        }
+        (void)split_row_active(a, row, k, p);
+        // steps: keys, then a scatter for each pass with a count between, the
+        // items' bounds, starts and exps, the denominator's maps
+        bool wide = false;
+        switch (step) {
+            case 0: split_keys<true>(a, t, T, row, p, 1, sh.keys); wide = true; break;
+            case 1: case 3: case 5: case 7:
+                split_scatter<true>(a, t, T, row, 4 * (step - 1), (step >> 1) & 1, 0, sh.scatter);
+                break;
+            case 2: case 4: case 6:
+                split_count<true>(a, t, T, row, 4 * step, (step >> 1) & 1, sh.count);
+                wide = true;
+                break;
+            case 8: split_bounds<true>(a, t, T, row, sh.bounds); break;
+            case 9: split_istart<true>(a, t, T, row, sh.istart); break;
+            case 10: split_exps<true>(a, t, T, row, p, k, sh.exps); wide = true; break;
+            default:
+                left_maps(a, row, t * kMapSub, (t + 1) * kMapSub, sh);
+                continue;  // (the last step: nothing waits for it)
+        }
+        // (every wave's stores are done before the tile is counted)
+        stores_done_barrier();
+        if (!wide) {
+            if (tid == 0) (void)__hip_atomic_fetch_add(progress, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            continue;
+        }
+        if (tid == 0) sh.go = __hip_atomic_fetch_add(progress, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        __syncthreads();
+        if (sh.go != need + static_cast<uint32_t>(T)) continue;
+        if (step < kLeftSteps - 2) split_scan<true>(a, T, row, sh.scan);
+        else if (wave == 0) split_meta<true>(a, T, row);
+        stores_done_barrier();
+        if (tid == 0) (void)__hip_atomic_fetch_add(progress, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -1996,7 +2268,10 @@ __global__ __launch_bounds__(kDThreads, kSorted ? 2 : 4) void fo_decide_kernel(D
         if (tid == 0 && !a.fo_fallback) skipped_row(a, row);
         return;
     }
-    if (a.fo_fallback && a.fo_meta[static_cast<int64_t>(row) * kMetaWords + kMetaStatus] != kStatusFallback) return;
+    if (a.fo_fallback) {
+        const uint32_t st = a.fo_meta[static_cast<int64_t>(row) * kMetaWords + kMetaStatus];
+        if (st != kStatusFallback && st != kStatusToSort) return;
+    }
 
     const int32_t* hist;
     int H;
@@ -2019,6 +2294,11 @@ __global__ __launch_bounds__(kDThreads, kSorted ? 2 : 4) void fo_decide_kernel(D
         }
         if (tid == 0) emit_row(a, row, token, prob, flags);
     };
+    if (a.fo_fallback && meta[kMetaStatus] == kStatusToSort) {
+        // fo_left_kernel's wait for the row's tiles ran out
+        finish(-1, 0.0f, GE_FLAG_TIMEOUT);
+        return;
+    }
     if (meta[kMetaStatus] != (a.fo_fallback ? kStatusFallback : kStatusOk)) {
         // Too many unique penalised ids for the extras: the fallback pass
         // re-samples the row (the caller launches it whenever a history may
@@ -3140,6 +3420,12 @@ hipError_t split_sort_f32(const DevArgs& s, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Whether a row's maps fit its share of the tile area and the decide kernel's staging.
+bool maps_fit(int vocab) {
+    return map_row_words(vocab) <= fo_tile_words(fo_split_tiles(vocab)) &&
+           (vocab + kMapTile - 1) / kMapTile * kMapSub * (kMapPartWords + 1) + 8 <= kFoExtrasCap;
+}
+
 template <typename T>
 hipError_t sorted_pass(const DevArgs& a, hipStream_t stream) {
     const int64_t stride = fo_items_stride_f32(a.vocab);
@@ -3150,9 +3436,11 @@ hipError_t sorted_pass(const DevArgs& a, hipStream_t stream) {
     // 1024 < top_k < V go to them straight away.
     const bool binned = std::is_same<T, float>::value && !a.fo_fallback && a.fo_tiles != nullptr &&
                         (a.row_params || a.params.top_k == 0u || a.params.top_k >= static_cast<uint32_t>(a.vocab)) &&
-                        a.fo_tiles_words >= fb_row_words(a.vocab);
+                        a.fo_tiles_words >= std::max(fb_row_words(a.vocab), fo_tile_words(fo_split_tiles(a.vocab)));
     if (binned) {
-        per64 = std::min(per64, a.fo_tiles_words / fb_row_words(a.vocab));
+        const int tiles = fo_split_tiles(a.vocab);
+        per64 = std::min({per64, a.fo_tiles_words / std::max(fb_row_words(a.vocab), fo_tile_words(tiles)),
+                          static_cast<int64_t>(64 * kLeftMasks)});
         for (int r0 = 0; r0 < a.rows; r0 += static_cast<int>(per64)) {
             DevArgs s = slice_rows(a, r0, static_cast<int>(std::min<int64_t>(per64, a.rows - r0)));
             s.fo_items_stride = stride;
@@ -3160,8 +3448,9 @@ hipError_t sorted_pass(const DevArgs& a, hipStream_t stream) {
             hipError_t e = launch_binned(s, stream);
             if (e != hipSuccess) return e;
             s.fo_fallback = 1;
-            s.fo_maps = 0;
-            hipLaunchKernelGGL(fo_sort_kernel<T>, dim3(s.rows), dim3(kThreads), 0, stream, s);
+            s.fo_maps = maps_fit(a.vocab) ? 1 : 0;
+            // one workgroup per CU, or per tile of fewer
+            hipLaunchKernelGGL(fo_left_kernel, dim3(std::min(256, s.rows * tiles)), dim3(kKThreads), 0, stream, s);
             hipLaunchKernelGGL((fo_decide_kernel<T, true>), dim3(s.rows), dim3(kDThreads), 0, stream, s);
             e = hipGetLastError();
             if (e != hipSuccess) return e;
@@ -3179,10 +3468,9 @@ hipError_t sorted_pass(const DevArgs& a, hipStream_t stream) {
                        per64 <= kSplitMaxRows && per64 * fo_tile_words(fo_split_tiles(a.vocab)) <= a.fo_tiles_words;
     const int per = static_cast<int>(std::max<int64_t>(1, per64));
     // The denominator's tile maps go to the tile area when it holds a slice.
-    const bool maps = a.fo_tiles != nullptr && map_row_words(a.vocab) <= fo_tile_words(fo_split_tiles(a.vocab)) &&
+    const bool maps = a.fo_tiles != nullptr && maps_fit(a.vocab) &&
                       static_cast<int64_t>(per) * fo_tile_words(fo_split_tiles(a.vocab)) <= a.fo_tiles_words &&
-                      per <= kMapRowGroups * 64 &&
-                      (a.vocab + kMapTile - 1) / kMapTile * kMapSub * (kMapPartWords + 1) + 8 <= kFoExtrasCap;
+                      per <= kMapRowGroups * 64;
     for (int r0 = 0; r0 < a.rows; r0 += per) {
         DevArgs s = slice_rows(a, r0, std::min(per, a.rows - r0));
         s.fo_items_stride = stride;

@@ -96,7 +96,7 @@ struct DevArgs {
 constexpr int kFoBins = 65536;                 // bf16 order keys
 constexpr int kFoNonNanBins = 65536 - 254;     // bf16 patterns that are not NaN
 constexpr int kFoExtrasCap = 8192;             // penalised tokens per row it handles
-constexpr int kMetaWords = 8;                  // per-row words of fo_meta
+constexpr int kMetaWords = 10;                // per-row words of fo_meta
 
 inline int64_t fo_items_stride(int max_history) {
     const int64_t extras = max_history < kFoExtrasCap ? (max_history > 0 ? max_history : 0) : kFoExtrasCap;
