@@ -644,8 +644,7 @@ __device__ __forceinline__ void fb_plan(const DevArgs& a, int row, int parts, Pl
         // and whatever the sum: it neither changes binade nor stops there. So
         // masked tokens and the tail of an open nucleus need no replay, however
         // many they are; every later bin is such a one too.
-        // (half an ulp, 2^(e - 151), as a float's bits: e is at least 67 here)
-        const bool none = f2u(qh) < static_cast<uint32_t>(max(ea, e_first) - 24) << 23;
+        const bool none = __builtin_ldexpf(qh, 150 - max(ea, e_first)) < 0.5f;
         // (the cut's bin: only where its tokens lie on both sides of the cut)
         const bool split = static_cast<uint32_t>(b) == cut && qh >= minimum;
         const bool kept = static_cast<uint32_t>(b) < cut || split;
