@@ -116,7 +116,10 @@ constexpr int64_t fo_tile_words(int tiles) { return static_cast<int64_t>(tiles) 
 // per row, is on the critical path (one row of V = 262,144: plan 36 -> 23 us,
 // order 6 -> 13; 64 rows 41 -> 26 and 19 -> 14), while many near-uniform rows
 // pay for the tokens of wider bins (256 rows: collect, order and draw 286 -> 363
-// us, plan 56 -> 37). And the words of a row's area in fo_tiles.
+// us, plan 56 -> 37). Whole calls with 16,384 and 8,192 bins: near-uniform rows of
+// V = 262,144, 96 rows 337 and 352 us, 128 363 and 384, 256 535 and 588; but of
+// V = 131,072, 256 rows, 386 and 378, and rows of normal logits, 128 and 256 rows,
+// 394 and 363, 586 and 553. And the words of a row's area in fo_tiles.
 constexpr int kFbMaxBins = 16384;
 constexpr int kFbParts = 64;    // workgroups that stream one row, at most
 constexpr int kFbSegs = 4096;   // expanded bins of one row, at most

@@ -2863,8 +2863,11 @@ __device__ __forceinline__ uint32_t pl_entries(uint32_t nl) {
 // Deterministic, so every workgroup of a row agrees.
 __device__ __forceinline__ uint32_t pl_rank(uint32_t k, int cpr, uint32_t entries) {
     const float mu = spec_mu(k, cpr);
-    // (few chunks: each holds a larger share of the top k, and 2 sqrt(mu) left
-    // 1 row in 30 short at 2 chunks, k = 64; 2.5 leaves 1 in 500)
+    // (Few chunks: where the last is nearly empty, the others hold more of the top
+    // k than mu. Simulated, k = 64, rows left short per 10,000 with 2 and with 2.5:
+    // V = 17,000 2,771 and 896, 20,000 262 and 25, 50,257 37 and 2; with full
+    // chunks none either way. Lists overflow a little more often, 0.5% and 0.8% at
+    // V = 20,000, which the wave mends itself.)
     const float dev = cpr <= 4 ? 2.5f : 2.0f;
     const uint32_t q = static_cast<uint32_t>(ceilf((mu + dev * __builtin_amdgcn_sqrtf(mu) + 4.0f) * 0.25f));
     return min(max(q, 1u), max(min(16u, entries / 2u), 1u));

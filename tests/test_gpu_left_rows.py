@@ -142,3 +142,20 @@ def test_replays_and_rings(sampler):
         assert_parity(w, tuple(o.cpu().numpy() for o in out[0]), first, "first call")
         assert_parity(w2, tuple(o.cpu().numpy() for o in out[1]), second, "second call")
         assert_parity(w, run_gpu(sampler, w), first, "between")
+
+
+@pytest.mark.parametrize("rows,vocab", [(3, 30000), (70, 30000), (2, W.VOCAB)])
+def test_denominators_to_replay(sampler, rows, vocab):
+    # the denominators' maps, of tiled rows and of rows with a workgroup each
+    from test_gpu_certificates import _on_a_boundary
+
+    rng = np.random.default_rng(vocab)
+    base = np.minimum(rng.standard_normal(vocab) * 3 - 14, -0.5)
+    base[0] = 0.0
+    row, rest, s = _on_a_boundary(base, "f32")
+    assert 0 <= rest < 500 * 2.0**-53 * s
+    x = np.stack([rng.permutation(row) for _ in range(rows)])
+    w = small_workload(f"replay-{rows}-{vocab}", x, dict(temperature=1.0, top_k=0, top_p=0.999), uniforms=W.mt_uniforms(4, rows))
+    print(f"[left] {w.name}", flush=True)
+    assert_parity(w, run_gpu(sampler, w), run_oracle(w))
+    assert rows_left(sampler, rows) == list(range(rows))
